@@ -416,7 +416,10 @@ sp::MoverParams mover_params(Ctx* c, double t0, double dtf, int num_fine_steps, 
     m.vdp_pre = (double)(1.0f / (float)(3 * f.charge));
     m.d1p0 = f.drift1 * f.p0;
     m.d2p02 = f.drift2 * (f.p0 * f.p0);
-    m.half_dx = 0.5 * f.dx; m.half_dy = 0.5 * f.dy; m.half_dz = 0.5 * f.dz;
+    const double half[3] = {0.5 * f.dx, 0.5 * f.dy, 0.5 * f.dz};
+    m.half_min = std::min(half[0], half[1]);
+    if (f.ndim == 3) m.half_min = std::min(m.half_min, half[2]);
+    m.inv_dtf = 1.0 / dtf;
     m.dt_min = f.dt_min_rel * dtf;  // set_dt_min_max (:5519-5524)
     m.dt_max = f.dt_max_rel * dtf;
     m.f_gs1 = 1.0f / c->gscale[0];
@@ -430,7 +433,7 @@ sp::MoverParams mover_params(Ctx* c, double t0, double dtf, int num_fine_steps, 
     m.f_vdp_pre = 1.0f / (float)(3 * f.charge);
     m.f_d1p0 = (float)m.d1p0;
     m.f_d2p02 = (float)m.d2p02;
-    m.f_half_dx = (float)m.half_dx; m.f_half_dy = (float)m.half_dy; m.f_half_dz = (float)m.half_dz;
+    m.f_half_dx = (float)half[0]; m.f_half_dy = (float)half[1]; m.f_half_dz = (float)half[2];
     m.f_dt_min = (float)m.dt_min;
     m.f_dt_max = (float)m.dt_max;
     m.inv_p0 = 1.0 / f.p0;

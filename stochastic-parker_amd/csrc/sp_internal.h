@@ -114,7 +114,7 @@ struct DevParams {
     int ndim;
     int nxg, nyg, nzg;
     double dx, dy, dz;
-    double idx, idy, idz;          // 1/dx ... (FP32 path only)
+    double idx, idy, idz;          // 1/dx ...
     double xmin, ymin, zmin, xmax, ymax, zmax;
     double lx, ly, lz;
     int pbc[3];
@@ -218,7 +218,7 @@ struct MoverParams {
     double t0, dtf, dt_fine, dt_limit;
     double xmin, ymin, zmin;
     double dx, dy, dz;            // FP64 path: p = (x - xmin) / dx
-    double idx, idy, idz;         // FP32 path: p = (x - xmin) * idx
+    double idx, idy, idz;         // FP32 path: p = (x - xmin) * idx; FP64: div_const
     double slo[3], shi[3];        // slack (half-cell) bounds used while stepping
     double elo[3], ehi[3];        // exact bounds of particle_mover's final pass
     double p0, p_floor;           // p_floor = 0.25 * p0
@@ -226,7 +226,8 @@ struct MoverParams {
     double kpara0, kret, pindex, gamma_m2;  // gamma_m2 = gamma_turb - 2
     double vdp_pre;               // (double)(1.0f / (3 * charge)), an FP32 quotient
     double d1p0, d2p02;           // drift1 * p0, drift2 * (p0 * p0)
-    double half_dx, half_dy, half_dz;
+    double half_min;              // smallest of the half cell widths of the ndim axes
+    double inv_dtf;
     double dt_min, dt_max;
     // FP32 physics
     float f_kpara0, f_kret, f_pindex, f_gm2, f_vdp_pre, f_d1p0, f_d2p02;

@@ -59,7 +59,7 @@ __device__ __forceinline__ void pin_constants(MoverParams& m) {
     pin_vgpr(m.p0); pin_vgpr(m.p_floor);
     pin_vgpr(m.kpara0); pin_vgpr(m.kret); pin_vgpr(m.pindex); pin_vgpr(m.gamma_m2);
     pin_vgpr(m.vdp_pre); pin_vgpr(m.d1p0); pin_vgpr(m.d2p02);
-    pin_vgpr(m.half_dx); pin_vgpr(m.half_dy); pin_vgpr(m.half_dz);
+    pin_vgpr(m.half_min); pin_vgpr(m.inv_dtf);
     pin_vgpr(m.dt_min); pin_vgpr(m.dt_max);
     pin_vgpr(m.f_kpara0); pin_vgpr(m.f_kret); pin_vgpr(m.f_pindex); pin_vgpr(m.f_gm2);
     pin_vgpr(m.f_vdp_pre); pin_vgpr(m.f_d1p0); pin_vgpr(m.f_d2p02);
