@@ -22,23 +22,21 @@ struct PolicyF64 {
         m.p0_2mpi = kv.p0_2mpi;
         m.perp_mag = kv.perp_mag; m.perp_mom = kv.perp_mom;
     }
-    // no records are kept across steps
     template <int NDIM, bool TI, int FX, int PPL>
-    struct Cache {
-        __device__ __forceinline__ void invalidate() {}
-    };
+    using Cache = f64::CellCache<NDIM == 3 && !TI && (FX & FX_DPP) == 0>;
     template <int NDIM, bool TI, int FX, class GC>
     __device__ __forceinline__ static void step(const MoverParams& m, const Var&, State& s,
                                                 bool fixed, uint32_t tagi, uint32_t tags,
-                                                uint32_t rstep, double d[4], GC&) {
+                                                uint32_t rstep, double d[4], GC& gc) {
         double r[4];
         f64::step_rands(m, tagi, tags, rstep, r);
-        f64::gather_kappa_push<NDIM, TI, FX>(m, s, fixed, r, d);
+        f64::gather_kappa_push<NDIM, TI, FX>(m, s, fixed, r, d, gc);
     }
     template <int NDIM, bool TI, int FX>
     __device__ __forceinline__ static void step_given(const MoverParams& m, const Var&, State& s,
                                                       bool fixed, const double* r, double d[4]) {
-        f64::gather_kappa_push<NDIM, TI, FX>(m, s, fixed, r, d);
+        f64::CellCache<false> none;
+        f64::gather_kappa_push<NDIM, TI, FX>(m, s, fixed, r, d, none);
     }
 };
 

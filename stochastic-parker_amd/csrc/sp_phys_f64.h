@@ -76,33 +76,93 @@ struct RecShape {
     static constexpr int NC = NDIM == 2 ? (DPP ? 18 : 15) : (DPP ? 28 : 21);
 };
 
-template <int NDIM, bool TINTERP, bool DPP = false>
+// The eight corner records of the cell a lane's particle last gathered from,
+// kept in registers across its steps (one-frame 3D steps without momentum
+// diffusion, at one wave per SIMD: 168 registers): the fields do not change
+// within a launch, so a step that starts in the same cell loads nothing (the
+// reference sums the corners in cell order, so records kept by node, as the
+// FP32 3D gather keeps them, would have to change places).  3e5 particles on
+// 64^3: 116 -> 103 ms of mover per interval.  Empty elsewhere: the 2D kernel's
+// two waves per SIMD leave no room for it.
+template <bool ON>
+struct CellCache {
+    static constexpr bool kOn = false;
+    __device__ __forceinline__ void invalidate() {}
+};
+template <>
+struct CellCache<true> {
+    static constexpr bool kOn = true;
+    float4 raw[8][kRec3D / 4 - 1];
+    float last[8];                // slot 20 (d|B|/dz); the rest is padding
+    long long key;                // record index of corner 0; -1: none
+    __device__ __forceinline__ void invalidate() { key = -1; }
+};
+
+template <int NDIM, bool TINTERP, bool DPP, class GC>
 __device__ __forceinline__ void gather(const MoverParams& m, const Interp& I, double rt,
-                                       double* __restrict__ f) {
+                                       double* __restrict__ f, GC& gc) {
     constexpr int W = RecShape<NDIM, DPP>::W;
     constexpr int NC = RecShape<NDIM, DPP>::NC;
     constexpr int NCORN = NDIM == 2 ? 4 : 8;
     double g[TINTERP ? NC : 1];
-    const long long sy = m.nxg, sz = (long long)m.nxg * m.nyg;
-    const long long base = (long long)I.ix + (long long)I.iy * sy + (long long)I.iz * sz;
+    // record index of corner q: in 3D brick_record as a sum of one part per
+    // axis and corner (the brick and the place in the brick), formed once
+    long long ax[2], ay[2], az[2];
+    if (NDIM == 3) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int ix = I.ix + e, iy = I.iy + e, iz = I.iz + e;
+            ax[e] = ((long long)(ix >> 3) << 9) | (ix & 7);
+            ay[e] = (((long long)(iy >> 3) * m.bnx) << 9) | ((iy & 7) << 3);
+            az[e] = (((long long)(iz >> 3) * m.bny * m.bnx) << 9) | ((iz & 7) << 6);
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            ax[e] = I.ix + e;
+            ay[e] = (long long)(I.iy + e) * m.nxg;
+            az[e] = 0;
+        }
+    }
+    auto corner = [&](int q) { return ax[q & 1] + ay[(q >> 1) & 1] + az[(q >> 2) & 1]; };
+    if constexpr (GC::kOn) {
+        static_assert(NDIM == 3 && !TINTERP && !DPP, "the cache holds 3D records of one frame");
+        const long long key = corner(0);
+        if (gc.key != key) {
+            gc.key = key;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const float* r = m.rec1 + corner(q) * W;
+#pragma unroll
+                for (int u = 0; u < W / 4 - 1; ++u) gc.raw[q][u] = reinterpret_cast<const float4*>(r)[u];
+                gc.last[q] = r[20];
+            }
+        }
+    }
 #pragma unroll
     for (int q = 0; q < NCORN; ++q) {
-        const int i = q & 1, j = (q >> 1) & 1, k = (q >> 2) & 1;
-        const long long node = NDIM == 3 ? brick_record(I.ix + i, I.iy + j, I.iz + k, m.bnx, m.bny)
-                                         : base + i + j * sy + k * sz;
-        const float4* r4 = reinterpret_cast<const float4*>(m.rec1 + node * W);
         float v[W];
+        if constexpr (GC::kOn) {
 #pragma unroll
-        for (int u = 0; u < W / 4; ++u) {
-            const float4 t = r4[u];
-            v[4 * u] = t.x; v[4 * u + 1] = t.y; v[4 * u + 2] = t.z; v[4 * u + 3] = t.w;
+            for (int u = 0; u < W / 4 - 1; ++u) {
+                const float4 t = gc.raw[q][u];
+                v[4 * u] = t.x; v[4 * u + 1] = t.y; v[4 * u + 2] = t.z; v[4 * u + 3] = t.w;
+            }
+            v[20] = gc.last[q];
+        } else {
+            const float4* r4 = reinterpret_cast<const float4*>(m.rec1 + corner(q) * W);
+#pragma unroll
+            for (int u = 0; u < W / 4; ++u) {
+                const float4 t = r4[u];
+                v[4 * u] = t.x; v[4 * u + 1] = t.y; v[4 * u + 2] = t.z; v[4 * u + 3] = t.w;
+            }
         }
         // the first corner starts the sums (0 + v w is v w but for a zero's sign)
         const double wq = I.w[q];
 #pragma unroll
         for (int c = 0; c < NC; ++c) f[c] = q == 0 ? (double)v[c] * wq : f[c] + (double)v[c] * wq;
         if (TINTERP) {
-            const float4* s4 = reinterpret_cast<const float4*>(m.rec2 + node * W);
+            const float4* s4 = reinterpret_cast<const float4*>(m.rec2 + corner(q) * W);
 #pragma unroll
             for (int u = 0; u < W / 4; ++u) {
                 const float4 t = s4[u];
@@ -493,14 +553,14 @@ __device__ __forceinline__ void step_rands(const MoverParams& m, uint32_t tag_i,
 }
 
 // The full per-step chain: interpolation parameters, gather, kappa, push.
-template <int NDIM, bool TINTERP, int FX>
+template <int NDIM, bool TINTERP, int FX, class GC>
 __device__ __forceinline__ void gather_kappa_push(const MoverParams& m, State& s, bool fixed_dt,
-                                                  const double r[4], double d[4]) {
+                                                  const double r[4], double d[4], GC& gc) {
     constexpr bool DPP = (FX & FX_DPP) != 0;
     double f[RecShape<NDIM, DPP>::NC];
     const Interp I = interp_params<NDIM>(m, s.x, s.y, s.z);
     const double rt = TINTERP ? div_const(s.t - m.t0, m.dtf, m.inv_dtf) : 0.0;
-    gather<NDIM, TINTERP, DPP>(m, I, rt, f);
+    gather<NDIM, TINTERP, DPP>(m, I, rt, f, gc);
     Kappa k;
     if constexpr ((FX & FX_NLGC) != 0) k = kappa_nlgc<NDIM>(m, s.p, s.mu, f);
     else k = kappa<NDIM>(m, s.p, f);

@@ -37,3 +37,24 @@ def test_step_without_powers_is_bit_exact(ndim, n, ti):
         row, dr = oracle.step_once(prm, fa[0], a[i], t0, dtf, fixed[i], r[i], *fa[1:])
         np.testing.assert_array_equal(st[i], [row[k] for k in COLS], err_msg=str(i))
         np.testing.assert_array_equal(d[i], dr, err_msg=str(i))
+
+
+@pytest.mark.parametrize("acc,mag", [(0, 0), (1, 1)])
+def test_3d_record_cache_changes_no_bit(acc, mag):
+    """A budget of one step per launch starts nearly every step with an empty
+    cache; without a budget a lane's records serve until the cell changes."""
+    c = cfg3d(13, pbcx=1, dt_max_rel=1e-3, acc_region_flag=acc, mag_dependency=mag,
+              acc_region=(0.1, 0.8, 0.2, 0.9, 0.0, 0.7))
+    out = []
+    for budget in (0, 1):
+        with ParkerPusher(**dict(c, precision="f64", nptl_max=4000, sort_steps=budget)) as pz:
+            pz.upload_fields(nodes_for(c), 0)
+            pz.calc_fields_gradients(0)
+            pz.inject_particles_spatial_uniform(3000, 1e-7, 1, 5.0, 0.0, 0.05, (0, 0, 0, 1, 1, 1))
+            st = pz.particle_mover(0.0, 0.05, 2, 10)
+            a = pz.get_particles()
+            o = np.argsort(a["tag_injected"])
+            out.append((st["steps"], {k: v[o] for k, v in a.items()}))
+    assert out[0][0] == out[1][0]
+    for k in out[0][1]:
+        np.testing.assert_array_equal(out[0][1][k], out[1][1][k], err_msg=k)
