@@ -667,6 +667,8 @@ __global__ void adamw_kernel(float* p, const float* gr, float* m, float* v, uint
 }  // namespace mlp
 }  // namespace sp
 
+#include "sp_mlp_train.h"
+
 // ---------------------------------------------------------------------------
 // Host side: the network context and the extern "C" entry points.
 namespace {
@@ -705,6 +707,11 @@ struct Mlp {
     float* ey = nullptr;                // outputs of device-array ensemble chunks
     long long ey_rows = 0;
     std::vector<hipEvent_t> tev;        // per-chunk timing events of the fused launches
+    // two-launch training steps: transposed weight fragments, the batch's
+    // activations and gradients, squared errors, loss partials per step
+    uint16_t *wb = nullptr, *xf = nullptr, *gf = nullptr;
+    float *sq = nullptr, *lparts = nullptr;
+    long long frag_rows = 0, lparts_steps = 0;
     long long step = 0;                 // AdamW step count
 };
 
@@ -724,7 +731,7 @@ void destroy(Mlp* n) {
     dfree(n->y); dfree(n->t); dfree(n->gh[0]); dfree(n->gh[1]); dfree(n->part);
     dfree(n->loss_hist); dfree(n->xin); dfree(n->xd); dfree(n->td); dfree(n->bidx);
     dfree(n->wpart); dfree(n->ens_spec); dfree(n->ens_spread); dfree(n->ts); dfree(n->wf);
-    dfree(n->ey);
+    dfree(n->ey); dfree(n->wb); dfree(n->xf); dfree(n->gf); dfree(n->sq); dfree(n->lparts);
     for (auto& e : n->ev)
         if (e) (void)hipEventDestroy(e);
     for (auto& e : n->tev)
@@ -786,6 +793,16 @@ int forward(Mlp* n, int rows, bool train = true) {
     return SP_OK;
 }
 
+// Rows per split of an M x N weight gradient over `rows` rows: up to 256
+// blocks of 128-wide tiles, at least 128 rows each.
+int wgrad_chunk(int M, int N, int rows) {
+    const int bn = N > 64 ? 128 : 64;
+    const int tiles = ((M + 127) / 128) * ((N + bn - 1) / bn);
+    int splits = std::max(1, std::min(kMaxSplits, 256 / std::max(1, tiles)));
+    splits = std::min(splits, (rows + 127) / 128);
+    return ((rows + splits - 1) / splits + 31) / 32 * 32;
+}
+
 // Loss, gradients of all parameters into n->g; the mean squared error goes to
 // loss_out (device), or with a training state to loss_out[t - t0].
 int backward(Mlp* n, int rows, float* loss_out, const sp::mlp::TrainState* ts = nullptr) {
@@ -809,12 +826,8 @@ int backward(Mlp* n, int rows, float* loss_out, const sp::mlp::TrainState* ts = 
         w.A = n->xh[l]; w.lda = n->K[l]; w.transA = 1;
         w.B = n->gh[cur]; w.ldb = n->N[l];
         w.M = n->K[l]; w.N = n->N[l]; w.K = rows;
-        const int bn = w.N > 64 ? 128 : 64;
-        const int tiles = ((w.M + 127) / 128) * ((w.N + bn - 1) / bn);
-        int splits = std::max(1, std::min(kMaxSplits, 256 / std::max(1, tiles)));
-        splits = std::min(splits, (rows + 127) / 128);
-        w.kchunk = ((rows + splits - 1) / splits + 31) / 32 * 32;
-        splits = (rows + w.kchunk - 1) / w.kchunk;
+        w.kchunk = wgrad_chunk(w.M, w.N, rows);
+        const int splits = (rows + w.kchunk - 1) / w.kchunk;
         const long long mn = (long long)w.M * w.N;
         w.outF = n->wpart;
         MLP_HIP(sp::mlp::gemm<sp::mlp::EPI_PLAIN>(w, n->st, splits));
@@ -951,6 +964,100 @@ int fused_forward(Mlp* const* ms, int members, const float* x, int rows, hipStre
     else if (H == 128 && NO == 64) launch_fused<128, 64>(a, members, s);
     else if (H == 128 && NO == 32) launch_fused<128, 32>(a, members, s);
     else launch_fused<128, 128>(a, members, s);
+    MLP_HIP(hipGetLastError());
+    return SP_OK;
+}
+
+// nsteps training steps of two launches each (sp_mlp_train.h); step s draws its
+// rows and its learning rate from s.  The losses end in n->loss_hist.
+bool train_fused_ok(const Mlp* n) {
+    return fused_ok(n) && n->cfg.nlayers <= sp::mlp::kTrainMaxHidden;
+}
+
+template <int H>
+void launch_train_rows(const sp::mlp::RowsArgs& a, int nl, unsigned grid, hipStream_t s) {
+    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(grid), dim3(2 * H), 0, s, a); };
+    if (nl == 1) go(sp::mlp::train_rows_kernel<H, 1>);
+    else if (nl == 2) go(sp::mlp::train_rows_kernel<H, 2>);
+    else if (nl == 3) go(sp::mlp::train_rows_kernel<H, 3>);
+    else if (nl == 4) go(sp::mlp::train_rows_kernel<H, 4>);
+    else go(sp::mlp::train_rows_kernel<H, 5>);
+}
+
+int train_fused(Mlp* n, int64_t nsteps, int batch, double lr0, double lr_min, uint64_t seed) {
+    static_assert(sp::mlp::kUpdateSplits == kMaxSplits && sp::mlp::kLossParts == kPartBlocks, "layer path's orders");
+    const sp_mlp_config& c = n->cfg;
+    const int H = c.nhidden, nl = c.nlayers, L = n->L;
+    const long long rows = (batch + 31) / 32 * 32;
+    const sp::mlp::RowFrags fr{(int)(rows / 16), H / 32};
+    if (!n->wb) MLP_HIP(hipMalloc(&n->wb, 2 * (size_t)nl * H * H));
+    if (n->frag_rows < rows) {
+        dfree(n->xf); dfree(n->gf); dfree(n->sq);
+        n->xf = n->gf = nullptr;
+        n->sq = nullptr;
+        n->frag_rows = 0;
+        MLP_HIP(hipMalloc(&n->xf, 2 * (size_t)fr.x(L)));
+        MLP_HIP(hipMalloc(&n->gf, 2 * (size_t)(fr.g(nl) + 16ll * fr.rs * c.nout)));
+        MLP_HIP(hipMalloc(&n->sq, 4 * (size_t)rows * c.nout));
+        n->frag_rows = rows;
+    }
+    if (n->lparts_steps < nsteps) {
+        dfree(n->lparts);
+        n->lparts = nullptr;
+        n->lparts_steps = 0;
+        // and the step's AdamW scalars behind the last partials
+        MLP_HIP(hipMalloc(&n->lparts, 4 * ((size_t)nsteps * sp::mlp::kLossParts + 4)));
+        n->lparts_steps = nsteps;
+    }
+    int rc = refresh_frag(n, n->st);
+    if (rc != SP_OK) return rc;
+    for (int l = 1; l < L; ++l) {
+        const long long cnt = (long long)n->K[l] * n->N[l];
+        hipLaunchKernelGGL(sp::mlp::frag_back_kernel, dim3(blocks(cnt)), dim3(256), 0, n->st,
+                           n->pb + n->woff[l], n->K[l], n->N[l], n->wb + (long long)(l - 1) * H * H);
+    }
+    MLP_HIP(hipGetLastError());
+    sp::mlp::RowsArgs ra{};
+    ra.xd = n->xd; ra.td = n->td;
+    ra.nd = (uint32_t)n->nd;
+    ra.k0 = (uint32_t)seed; ra.k1 = (uint32_t)(seed >> 32);
+    ra.rows = batch; ra.nin = c.nin; ra.nout = c.nout;
+    ra.fr = fr;
+    ra.wf = n->wf; ra.wb = n->wb;
+    ra.p = n->p;
+    ra.xf = n->xf; ra.gf = n->gf; ra.sq = n->sq;
+    ra.scale = 1.0f / (float)((long long)batch * c.nout);
+    ra.adam = n->lparts + n->lparts_steps * sp::mlp::kLossParts;
+    sp::mlp::UpdateArgs ua{};
+    ua.adam = ra.adam;
+    ua.rows = batch; ua.nin = c.nin; ua.hidden = H; ua.nl = nl; ua.nout = c.nout;
+    ua.fr = fr;
+    ua.xf = n->xf; ua.gf = n->gf; ua.sq = n->sq;
+    ua.p = n->p; ua.m = n->m; ua.v = n->v; ua.pb = n->pb; ua.wf = n->wf; ua.wb = n->wb;
+    ra.nsteps = (uint32_t)nsteps;
+    ra.lr0 = (float)lr0; ra.lr_min = (float)lr_min;
+    ra.b1 = ua.b1 = (float)c.beta1;
+    ra.b2 = ua.b2 = (float)c.beta2;
+    ua.eps = (float)c.eps; ua.wd = (float)c.weight_decay;
+    unsigned grid = 0;
+    for (int l = 0; l < L; ++l) {
+        ra.boff[l] = ua.boff[l] = n->boff[l];
+        ua.woff[l] = n->woff[l];
+        ua.kchunk[l] = wgrad_chunk(n->K[l], n->N[l], batch);
+        grid += (unsigned)((n->K[l] + 31) / 32 * (n->N[l] / 32) + n->N[l] / 32);
+    }
+    for (int64_t s = 0; s < nsteps; ++s) {
+        ra.step = (uint32_t)s;
+        ra.t = (uint32_t)(n->step + s);
+        ua.loss_parts = n->lparts + s * sp::mlp::kLossParts;
+        if (H == 256) launch_train_rows<256>(ra, nl, (unsigned)(rows / 32), n->st);
+        else launch_train_rows<128>(ra, nl, (unsigned)(rows / 32), n->st);
+        hipLaunchKernelGGL(sp::mlp::train_update_kernel, dim3(grid), dim3(sp::mlp::kUpdateBlock), 0, n->st, ua);
+        MLP_HIP(hipGetLastError());
+    }
+    if (nsteps > 0)
+        hipLaunchKernelGGL(sp::mlp::train_loss_kernel, dim3((unsigned)nsteps), dim3(256), 0, n->st, n->lparts,
+                           ra.scale, n->loss_hist);
     MLP_HIP(hipGetLastError());
     return SP_OK;
 }
@@ -1340,7 +1447,11 @@ int sp_mlp_train(void* q, int64_t nsteps, int32_t batch, double lr0, double lr_m
     };
     const char* eager_env = std::getenv("SP_MLP_EAGER");
     const bool eager = eager_env && std::atoi(eager_env) != 0;
-    if (eager || nsteps < 2) {
+    if (!eager && train_fused_ok(n)) {
+        rc = train_fused(n, nsteps, batch, lr0, lr_min, seed);
+        if (rc != SP_OK) return rc;
+        n->fver = n->pver;   // the update kernel keeps wf with the weights
+    } else if (eager || nsteps < 2) {
         for (int64_t s = 0; s < nsteps; ++s) {
             rc = one_step();
             if (rc != SP_OK) return rc;
