@@ -85,7 +85,6 @@ struct Ctx {
     uint32_t* skey[2] = {nullptr, nullptr};
     uint32_t* sidx[2] = {nullptr, nullptr};
     unsigned* shist = nullptr;
-    unsigned long long* soff = nullptr;
     long long mover_calls = 0;
     // autotuned launch settings (0 / -1: not tuned) and the tuner's state copy
     int tuned_bpc = 0, tuned_sort_steps = -1;
@@ -308,9 +307,9 @@ int mover_grid(Ctx* c, long long n, int bpc = 0, int ppl = 1) {
 }
 
 // Orders the current particle set by the Morton key of 2^shift-cell blocks
-// (at most 64 blocks per axis) into the spare buffer set and swaps.  With
-// paused_first, only the first `n` particles are ordered, in place: those the
-// mover paused (rdt > 0) first, in key order, then the others.
+// (at most 64 blocks per axis), in place; the spare buffer set is scratch.  With
+// paused_first, only the first `n` particles are ordered: those the mover
+// paused (rdt > 0) first, in key order, then the others.
 int spatial_sort(Ctx* c, bool paused_first = false, long long n = -1) {
     if (n < 0) n = c->nptl;
     if (n <= 1) return SP_OK;
@@ -322,8 +321,7 @@ int spatial_sort(Ctx* c, bool paused_first = false, long long n = -1) {
             SP_HIP(hipMalloc(&c->skey[i], sizeof(uint32_t) * cap));
             SP_HIP(hipMalloc(&c->sidx[i], sizeof(uint32_t) * cap));
         }
-        SP_HIP(hipMalloc(&c->shist, sizeof(unsigned) * 16 * nt));
-        SP_HIP(hipMalloc(&c->soff, sizeof(unsigned long long) * 16 * nt));
+        SP_HIP(hipMalloc(&c->shist, sizeof(unsigned) * (1 << sp::kSortDigitBits) * (nt + 1)));
     }
     const sp_config& f = c->cfg;
     sp::SortArgs sa{};
@@ -338,14 +336,11 @@ int spatial_sort(Ctx* c, bool paused_first = false, long long n = -1) {
     if (axis_bits > (f.ndim == 3 ? 10 : 15)) return fail(SP_ERR_UNSUPPORTED, "sort key too wide");
     const int kbits = f.ndim * axis_bits + (paused_first ? 1 : 0);
     sa.done_bit = paused_first ? f.ndim * axis_bits : -1;
-    sa.passes = (kbits + 3) / 4;
+    sa.passes = (kbits + sp::kSortDigitBits - 1) / sp::kSortDigitBits;
     sa.xmin = f.xmin; sa.ymin = f.ymin; sa.zmin = f.zmin;
     sa.idx = 1.0 / f.dx; sa.idy = 1.0 / f.dy; sa.idz = 1.0 / f.dz;
-    const bool prefix = n < c->nptl;
-    SP_HIP(sp::launch_spatial_sort(c->P[c->cur], c->P[1 - c->cur], n, sa, c->skey[0],
-                                   c->sidx[0], c->skey[1], c->sidx[1], c->shist, c->soff,
-                                   c->totals, prefix, c->st));
-    if (!prefix) c->cur = 1 - c->cur;
+    SP_HIP(sp::launch_spatial_sort(c->P[c->cur], sp::PtlBase{static_cast<char*>(c->pbuf[1 - c->cur]), cap}, n,
+                                   sa, c->skey[0], c->sidx[0], c->skey[1], c->sidx[1], c->shist, c->st));
     return SP_OK;
 }
 
@@ -471,7 +466,6 @@ void destroy(Ctx* c) {
         free_dev(c->sidx[i]);
     }
     free_dev(c->shist);
-    free_dev(c->soff);
     free_dev(c->dglob);
     for (auto* q : c->dloc) free_dev(q);
     for (auto* q : c->desc) free_dev(q);
