@@ -206,6 +206,7 @@ struct MoverParams {
     long long n;
     long long part_len;           // particles per XCD part (the last part may be shorter)
     unsigned step_budget;         // steps per particle per launch before it pauses (0 = none)
+    const uint32_t* order;        // order in which the parts hand out particles (nullptr: by index)
     const KappaVar* var;          // per-variant diffusion parameters (nvar > 0)
     int nvar;                     // 0: every particle uses the values below
     const float* rec1;
@@ -278,5 +279,10 @@ hipError_t launch_step_once_f64(const MoverParams& m, bool ti, int fx, int ndim,
 hipError_t launch_step_once_f32(const MoverParams& m, bool ti, int fx, int ndim, double* state,
                                 const double* rands, const int8_t* fixed, double* deltas,
                                 hipStream_t s);
+
+// digit[i]: mover part and predicted step-count class of particle i
+hipError_t launch_order_digit_f64(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit, hipStream_t s);
+hipError_t launch_order_digit_f32(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit, hipStream_t s);
+hipError_t launch_order_digit_f32h(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit, hipStream_t s);
 
 }  // namespace sp

@@ -55,4 +55,8 @@ hipError_t launch_step_once_f64(const MoverParams& m, bool ti, int fx, int ndim,
     return launch_step_once<PolicyF64>(m, ti, fx, ndim, state, rands, fixed, deltas, s);
 }
 
+hipError_t launch_order_digit_f64(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit, hipStream_t s) {
+    return launch_order_digit<PolicyF64>(m, ti, fx, ndim, digit, s);
+}
+
 }  // namespace sp

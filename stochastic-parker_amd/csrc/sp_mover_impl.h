@@ -106,7 +106,9 @@ constexpr bool kTwoWavePair = NDIM == 2 && PPL == 2;
 template <class Pol, int NDIM, bool TINTERP, int PPL>
 constexpr bool kThreeWave = Pol::kThreeWave2D && NDIM == 2 && !TINTERP && PPL == 1;
 
-template <class Pol, int NDIM, bool TINTERP, int FX, int PPL>
+// ORDER: the parts hand out particles in the order of m.order (a kernel of its
+// own: the test and the pointer in the other kernels cost them 2-3 %).
+template <class Pol, int NDIM, bool TINTERP, int FX, int PPL, bool ORDER = false>
 __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(kThreeWave<Pol, NDIM, TINTERP, PPL> ? 3 : (kTwoWavePair<NDIM, PPL> ? 2 : 1),
                                    kThreeWave<Pol, NDIM, TINTERP, PPL> ? 3 : 2)))
@@ -181,9 +183,10 @@ mover_kernel(MoverParams m0) {
                 if (++parts_done == kParts) exhausted = true;
             }
             if (need) {
-                const long long j =
+                long long j =
                     pb + (long long)(base + (unsigned long long)__popcll(need_mask & ((1ull << lane) - 1ull)));
                 if (j < pe) {
+                    if constexpr (ORDER) j = m0.order[j];
                     q.idx = j;
                     if (k == 0) gc.invalidate();
                     q.s.x = px[j];
@@ -419,6 +422,29 @@ __global__ void __launch_bounds__(256) step_once_kernel(MoverParams m, double* s
     for (int c = 0; c < 4; ++c) deltas[4 * i + c] = d[c];
 }
 
+// Part of each particle (m.part_len) and the class of the step count that its
+// first step's dt predicts, the larger counts first: classes a factor of two
+// apart from the smallest count, dtf / dt_max, up.  digit = part * 8 + class.
+constexpr int kOrderClasses = 8;
+template <class Pol, int NDIM, bool TINTERP, int FX>
+__global__ void __launch_bounds__(256) order_digit_kernel(MoverParams m, uint32_t* digit) {
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= m.n) return;
+    State s{m.P.d(PD_X)[i], m.P.d(PD_Y)[i], m.P.d(PD_Z)[i], m.P.d(PD_P)[i], m.P.d(PD_T)[i], m.P.d(PD_DT)[i], 0.0};
+    if constexpr ((FX & FX_NLGC) != 0) s.mu = m.P.d(PD_MU)[i];
+    typename Pol::Var var = Pol::var_of(m);
+    if (m.nvar > 0) {
+        const int v = m.P.i(PI_ORIGIN)[i];
+        Pol::set_var(m, var, m.var[v < 0 ? 0 : (v >= m.nvar ? m.nvar - 1 : v)]);
+    }
+    const double still[4] = {0.0, 0.0, 0.0, 0.0};
+    double d[4];
+    Pol::template step_given<NDIM, TINTERP, FX>(m, var, s, false, still, d);
+    const float c = __builtin_amdgcn_logf((float)m.dt_max / (float)s.dt);   // log2; a NaN goes last
+    const int few = c > 0.0f ? (int)fminf(c, (float)(kOrderClasses - 1)) : 0;
+    digit[i] = (uint32_t)(i / m.part_len) * kOrderClasses + (uint32_t)(kOrderClasses - 1 - few);
+}
+
 template <int N, bool T, int X>
 struct Variant {
     static constexpr int ndim = N;
@@ -489,18 +515,45 @@ int mover_occupancy(int ndim, bool ti, int fx, int ppl) {
     });
 }
 
+// Whether the mover and the digits for a work order are built: one-frame 2D
+// steps without acceleration region, momentum diffusion or NLGC.
+template <class V>
+constexpr bool kOrdered = V::ndim == 2 && !V::ti && (V::fx & ~FX_LEAN) == 0;
+
 template <class Pol>
 hipError_t launch_mover(const MoverParams& m, bool ti, int fx, int ndim, int ppl, int grid,
                         hipStream_t st) {
-    dispatch_variant<Pol>(ndim, ti, fx, [&](auto v) {
+    const int built = dispatch_variant<Pol>(ndim, ti, fx, [&](auto v) {
         return dispatch_ppl<Pol>(ppl, v, [&](auto vv, auto pc) {
             using V = decltype(vv);
-            hipLaunchKernelGGL((mover_kernel<Pol, V::ndim, V::ti, V::fx, decltype(pc)::value>),
-                               dim3(grid), dim3(256), 0, st, m);
-            return 0;
+            constexpr int kPpl = decltype(pc)::value;
+            if (m.order) {
+                if constexpr (kOrdered<V> && kPpl == 1)
+                    hipLaunchKernelGGL((mover_kernel<Pol, V::ndim, V::ti, V::fx, 1, true>), dim3(grid),
+                                       dim3(256), 0, st, m);
+                return kOrdered<V> && kPpl == 1 ? 1 : 0;
+            }
+            hipLaunchKernelGGL((mover_kernel<Pol, V::ndim, V::ti, V::fx, kPpl>), dim3(grid), dim3(256), 0, st,
+                               m);
+            return 1;
         });
     });
-    return hipGetLastError();
+    return built ? hipGetLastError() : hipErrorInvalidValue;
+}
+
+template <class Pol>
+hipError_t launch_order_digit(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit,
+                              hipStream_t st) {
+    if (m.n <= 0) return hipSuccess;
+    const int grid = (int)((m.n + 255) / 256);
+    const int built = dispatch_variant<Pol>(ndim, ti, fx, [&](auto v) {
+        using V = decltype(v);
+        if constexpr (kOrdered<V>)
+            hipLaunchKernelGGL((order_digit_kernel<Pol, V::ndim, V::ti, V::fx>), dim3(grid), dim3(256), 0, st,
+                               m, digit);
+        return kOrdered<V> ? 1 : 0;
+    });
+    return built ? hipGetLastError() : hipErrorInvalidValue;
 }
 
 template <class Pol>

@@ -73,6 +73,9 @@ hipError_t launch_copy(const void* a, void* b, long long n16, hipStream_t s);
 hipError_t launch_spatial_sort(const Ptl& P, const PtlBase& spare, long long n, const SortArgs& sa,
                                uint32_t* keyA, uint32_t* idxA, uint32_t* keyB, uint32_t* idxB,
                                unsigned* hist, hipStream_t s);
+// order = the indices 0 .. n - 1 by digit (below 64), stable; hist as above.
+hipError_t launch_digit_order(const uint32_t* digit, long long n, uint32_t* order, unsigned* hist,
+                              hipStream_t s);
 hipError_t launch_inject(const DevParams& prm, const Ptl& P, long long start, long long nptl,
                          long long nmax, int tag0, const InjectArgs& ia, hipStream_t s);
 hipError_t launch_threshold_count(const DevParams& prm, const ThreshArgs& ta,

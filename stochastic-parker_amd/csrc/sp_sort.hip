@@ -250,6 +250,18 @@ __global__ void __launch_bounds__(kBlock) unpack_rows_kernel(Rows R, Ptl D, long
 
 }  // namespace
 
+hipError_t launch_digit_order(const uint32_t* digit, long long n, uint32_t* order, unsigned* hist,
+                              hipStream_t s) {
+    if (n <= 0) return hipSuccess;
+    const long long ntiles = num_tiles(n);
+    unsigned* totals = hist + kDigits * ntiles;
+    hipLaunchKernelGGL(digit_count_kernel, dim3((unsigned)ntiles), dim3(kBlock), 0, s, digit, n, 0, ntiles, hist);
+    hipLaunchKernelGGL(digit_scan_kernel, dim3(kDigits), dim3(kScanBlock), 0, s, hist, ntiles, totals);
+    hipLaunchKernelGGL(digit_scatter_kernel, dim3((unsigned)ntiles), dim3(kBlock), 0, s, digit,
+                       (const uint32_t*)nullptr, (uint32_t*)nullptr, order, n, 0, ntiles, hist, totals);
+    return hipGetLastError();
+}
+
 hipError_t launch_spatial_sort(const Ptl& P, const PtlBase& spare, long long n, const SortArgs& sa,
                                uint32_t* keyA, uint32_t* idxA, uint32_t* keyB, uint32_t* idxB,
                                unsigned* hist, hipStream_t s) {
