@@ -23,6 +23,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstdlib>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -668,6 +669,7 @@ __global__ void adamw_kernel(float* p, const float* gr, float* m, float* v, uint
 }  // namespace sp
 
 #include "sp_mlp_train.h"
+#include "sp_mlp_query.h"
 
 // ---------------------------------------------------------------------------
 // Host side: the network context and the extern "C" entry points.
@@ -712,10 +714,21 @@ struct Mlp {
     uint16_t *wb = nullptr, *xf = nullptr, *gf = nullptr;
     float *sq = nullptr, *lparts = nullptr;
     long long frag_rows = 0, lparts_steps = 0;
+    char* pin = nullptr;                // pinned host staging of small queries (kPinBytes)
     long long step = 0;                 // AdamW step count
 };
 
 constexpr int kPartBlocks = 256;
+// Query rows that go to the one-launch kernel: at most one 32-row block per CU;
+// with more rows its blocks re-read the weights where the 128-row blocks of the
+// inference kernel do so a quarter as often.  Two members of 256 x 4, host
+// arrays: 8 rows 75 -> 40 us, 2000 rows 118 -> 67, 8000 rows 216 -> 202; device
+// arrays: 8192 rows 47 -> 36.
+constexpr int64_t kQueryRowsMax = 8192;
+// Rows and results of up to this size together go through pinned host memory,
+// which the kernel reads and writes itself: without it 940 rows take 89 us
+// instead of 55, 8000 rows 207 instead of 202.
+constexpr size_t kPinBytes = 5 << 19;
 constexpr int kMaxSplits = 32;
 
 void dfree(void* q) {
@@ -732,6 +745,7 @@ void destroy(Mlp* n) {
     dfree(n->loss_hist); dfree(n->xin); dfree(n->xd); dfree(n->td); dfree(n->bidx);
     dfree(n->wpart); dfree(n->ens_spec); dfree(n->ens_spread); dfree(n->ts); dfree(n->wf);
     dfree(n->ey); dfree(n->wb); dfree(n->xf); dfree(n->gf); dfree(n->sq); dfree(n->lparts);
+    if (n->pin) (void)hipHostFree(n->pin);
     for (auto& e : n->ev)
         if (e) (void)hipEventDestroy(e);
     for (auto& e : n->tev)
@@ -939,23 +953,30 @@ void launch_fused(const sp::mlp::FusedArgs& a, int members, hipStream_t s) {
     hipLaunchKernelGGL((sp::mlp::mlp_infer_kernel<H, NOUT, sp::mlp::kFusedRows / 32>), grid, dim3(2 * H), 0, s, a);
 }
 
+// Kernel arguments of the fused networks, without rows, x and y.
+sp::mlp::FusedArgs fused_args(Mlp* const* ms, int members) {
+    const Mlp* h = ms[0];
+    sp::mlp::FusedArgs a{};
+    a.nin = h->cfg.nin;
+    a.nhh = h->L - 2;
+    for (int i = 0; i < members; ++i) {
+        a.wf[i] = ms[i]->wf;
+        a.p[i] = ms[i]->p;
+    }
+    for (int l = 0; l < h->L; ++l) a.boff[l] = h->boff[l];
+    return a;
+}
+
 // y[i] (rows x nout; ms[i]->y when y is NULL) = network i (x), all members
 // in one launch on s.  Needs fused_ok and equal shapes, and every member's wf
 // refreshed.
 int fused_forward(Mlp* const* ms, int members, const float* x, int rows, hipStream_t s,
                   float* const* y = nullptr) {
     const Mlp* h = ms[0];
-    sp::mlp::FusedArgs a{};
+    sp::mlp::FusedArgs a = fused_args(ms, members);
     a.x = x;
     a.rows = rows;
-    a.nin = h->cfg.nin;
-    a.nhh = h->L - 2;
-    for (int i = 0; i < members; ++i) {
-        a.wf[i] = ms[i]->wf;
-        a.p[i] = ms[i]->p;
-        a.y[i] = y ? y[i] : ms[i]->y;
-    }
-    for (int l = 0; l < h->L; ++l) a.boff[l] = h->boff[l];
+    for (int i = 0; i < members; ++i) a.y[i] = y ? y[i] : ms[i]->y;
     if (rows == 0) return SP_OK;
     const int H = h->cfg.nhidden, NO = h->cfg.nout;
     if (H == 256 && NO == 64) launch_fused<256, 64>(a, members, s);
@@ -1084,6 +1105,57 @@ bool device_memory(const void* q) {
     return at.type == hipMemoryTypeDevice || at.type == hipMemoryTypeManaged;
 }
 
+// Ensemble spectra of up to kQueryRowsMax rows in one launch; the members' wf
+// are refreshed and their streams idle.
+int query(Mlp* const* ms, int members, const float* x, int rows, double floor, float* spec,
+          float* spread, bool dev) {
+    Mlp* h = ms[0];
+    const size_t nx = 4 * (size_t)rows * h->cfg.nin, ny = 4 * (size_t)rows * h->cfg.nout, nr = 4 * (size_t)rows;
+    const bool pinned = !dev && nx + ny + nr <= kPinBytes;
+    sp::mlp::QueryArgs a{};
+    a.f = fused_args(ms, members);
+    a.f.rows = rows;
+    a.members = members;
+    a.nout = h->cfg.nout;
+    a.floor = (float)floor;
+    a.f.x = x;
+    a.spec = spec;
+    a.spread = spread;
+    if (pinned) {
+        if (!h->pin) MLP_HIP(hipHostMalloc(reinterpret_cast<void**>(&h->pin), kPinBytes, hipHostMallocDefault));
+        a.spec = reinterpret_cast<float*>(h->pin);           // 16-byte rows first
+        a.spread = reinterpret_cast<float*>(h->pin + ny);
+        float* px = reinterpret_cast<float*>(h->pin + ny + nr);
+        std::memcpy(px, x, nx);
+        a.f.x = px;
+    } else if (!dev) {
+        MLP_HIP(hipMemcpyAsync(h->xin, x, nx, hipMemcpyHostToDevice, h->st));
+        a.f.x = h->xin;
+        a.spec = h->ens_spec;
+        a.spread = h->ens_spread;
+    }
+    MLP_HIP(hipEventRecord(h->tev[0], h->st));
+    const dim3 grid((unsigned)((rows + sp::mlp::kQueryRows - 1) / sp::mlp::kQueryRows));
+    const dim3 block((unsigned)(2 * h->cfg.nhidden * members));
+    if (h->cfg.nhidden == 256) hipLaunchKernelGGL(sp::mlp::mlp_query_kernel<256>, grid, block, 0, h->st, a);
+    else hipLaunchKernelGGL(sp::mlp::mlp_query_kernel<128>, grid, block, 0, h->st, a);
+    MLP_HIP(hipGetLastError());
+    MLP_HIP(hipEventRecord(h->tev[1], h->st));
+    if (!dev && !pinned) {
+        MLP_HIP(hipMemcpyAsync(spec, h->ens_spec, ny, hipMemcpyDeviceToHost, h->st));
+        MLP_HIP(hipMemcpyAsync(spread, h->ens_spread, nr, hipMemcpyDeviceToHost, h->st));
+    }
+    MLP_HIP(hipStreamSynchronize(h->st));
+    if (pinned) {
+        std::memcpy(spec, a.spec, ny);
+        std::memcpy(spread, a.spread, nr);
+    }
+    float t = 0.f;
+    MLP_HIP(hipEventElapsedTime(&t, h->tev[0], h->tev[1]));
+    h->fwd_ms = t;
+    return SP_OK;
+}
+
 int ensemble(void* const* nets, int32_t members, const float* x, int64_t rows, double floor,
              float* spec, float* spread, bool dev) {
     if (!nets || members < 1 || members > 8) return sp::set_error(SP_ERR_ARG, "members must be in [1, 8]");
@@ -1107,6 +1179,8 @@ int ensemble(void* const* nets, int32_t members, const float* x, int64_t rows, d
         fused = fused && fused_ok(n) && same_shape(n, h);
     }
     const int nin = h->cfg.nin, nout = h->cfg.nout;
+    const bool small = fused && rows > 0 && rows <= kQueryRowsMax && (dev || rows <= chunk) &&
+                       2 * h->cfg.nhidden * members <= sp::mlp::kQueryThreads;
     if (!dev && !h->ens_spec) {
         MLP_HIP(hipMalloc(&h->ens_spec, 4 * (size_t)h->bmax * nout));
         MLP_HIP(hipMalloc(&h->ens_spread, 4 * (size_t)h->bmax));
@@ -1115,7 +1189,7 @@ int ensemble(void* const* nets, int32_t members, const float* x, int64_t rows, d
     // own output buffers (fewer, fuller launches than batch_max-row chunks)
     std::vector<float*> ys((size_t)members, nullptr);
     for (int i = 0; i < members; ++i) ys[(size_t)i] = ms[(size_t)i]->y;
-    if (dev && fused && rows > 0) {
+    if (dev && fused && rows > 0 && !small) {
         chunk = (int)std::min<int64_t>(rows, (int64_t)1 << 20);
         for (int i = 0; i < members; ++i) {
             Mlp* n = ms[(size_t)i];
@@ -1139,6 +1213,7 @@ int ensemble(void* const* nets, int32_t members, const float* x, int64_t rows, d
         rc = ensure_events(h, 2 * (size_t)nchunks);
         if (rc != SP_OK) return rc;
     }
+    if (small) return query(ms.data(), members, x, (int)rows, floor, spec, spread, dev);
     for (int64_t c = 0; c < nchunks; ++c) {
         const int64_t r0 = c * chunk;
         const int r = (int)std::min<int64_t>(chunk, rows - r0);
