@@ -253,6 +253,19 @@ int set_error(int code, const std::string& msg);
 // Launchers (defined in the .hip translation units)
 hipError_t launch_gradients(const DevParams& prm, const float* nodes8, float* rec, float* farray32,
                             hipStream_t s);
+// Rows of a single-step launch, in up to kStagePieces pieces that lie apart:
+// state (6 doubles a row), random numbers and deltas (4), flags, the particle
+// whose mu row 0 takes with NLGC.
+constexpr int kStagePieces = 4;
+struct StepRows {
+    double* state[kStagePieces];
+    const double* rands[kStagePieces];
+    const int8_t* fixed[kStagePieces];
+    double* deltas[kStagePieces];
+    long long row0[kStagePieces];
+    long long n[kStagePieces];
+    int pieces;
+};
 // Records of the FP32 movers.  FP16 records: max |gradient| and max |V| of
 // the frame (as float bits, into maxbits[0] and maxbits[1]) set its
 // power-of-two scales, then the packing applies them.
@@ -264,8 +277,7 @@ hipError_t launch_pack_fast(const DevParams& prm, const float* nodes8, bool half
 int mover_blocks_per_cu_f32h(int ndim, bool ti, int fx, int ppl);
 hipError_t launch_mover_f32h(const MoverParams& m, bool ti, int fx, int ndim, int ppl, int grid,
                              hipStream_t s);
-hipError_t launch_step_once_f32h(const MoverParams& m, bool ti, int fx, int ndim, double* state,
-                                 const double* rands, const int8_t* fixed, double* deltas,
+hipError_t launch_step_once_f32h(const MoverParams& m, bool ti, int fx, int ndim, const StepRows& r,
                                  hipStream_t s);
 int mover_blocks_per_cu_f64(int ndim, bool ti, int fx);
 int mover_blocks_per_cu_f32(int ndim, bool ti, int fx, int ppl);
@@ -273,11 +285,9 @@ hipError_t launch_mover_f64(const MoverParams& m, bool ti, int fx, int ndim, int
                             hipStream_t s);
 hipError_t launch_mover_f32(const MoverParams& m, bool ti, int fx, int ndim, int ppl, int grid,
                             hipStream_t s);
-hipError_t launch_step_once_f64(const MoverParams& m, bool ti, int fx, int ndim, double* state,
-                                const double* rands, const int8_t* fixed, double* deltas,
+hipError_t launch_step_once_f64(const MoverParams& m, bool ti, int fx, int ndim, const StepRows& r,
                                 hipStream_t s);
-hipError_t launch_step_once_f32(const MoverParams& m, bool ti, int fx, int ndim, double* state,
-                                const double* rands, const int8_t* fixed, double* deltas,
+hipError_t launch_step_once_f32(const MoverParams& m, bool ti, int fx, int ndim, const StepRows& r,
                                 hipStream_t s);
 
 // digit[i]: mover part and predicted step-count class of particle i

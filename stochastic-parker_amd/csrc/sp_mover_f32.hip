@@ -76,10 +76,9 @@ hipError_t launch_mover_f32h(const MoverParams& m, bool ti, int fx, int ndim, in
     return launch_mover<PolicyF32H>(m, ti, fx, ndim, ppl, grid, s);
 }
 
-hipError_t launch_step_once_f32h(const MoverParams& m, bool ti, int fx, int ndim, double* state,
-                                 const double* rands, const int8_t* fixed, double* deltas,
+hipError_t launch_step_once_f32h(const MoverParams& m, bool ti, int fx, int ndim, const StepRows& r,
                                  hipStream_t s) {
-    return launch_step_once<PolicyF32H>(m, ti, fx, ndim, state, rands, fixed, deltas, s);
+    return launch_step_once<PolicyF32H>(m, ti, fx, ndim, r, s);
 }
 
 int mover_blocks_per_cu_f32(int ndim, bool ti, int fx, int ppl) {
@@ -91,10 +90,9 @@ hipError_t launch_mover_f32(const MoverParams& m, bool ti, int fx, int ndim, int
     return launch_mover<PolicyF32>(m, ti, fx, ndim, ppl, grid, s);
 }
 
-hipError_t launch_step_once_f32(const MoverParams& m, bool ti, int fx, int ndim, double* state,
-                                const double* rands, const int8_t* fixed, double* deltas,
+hipError_t launch_step_once_f32(const MoverParams& m, bool ti, int fx, int ndim, const StepRows& r,
                                 hipStream_t s) {
-    return launch_step_once<PolicyF32>(m, ti, fx, ndim, state, rands, fixed, deltas, s);
+    return launch_step_once<PolicyF32>(m, ti, fx, ndim, r, s);
 }
 
 hipError_t launch_order_digit_f32(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit, hipStream_t s) {

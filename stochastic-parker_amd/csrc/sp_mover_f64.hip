@@ -49,10 +49,9 @@ hipError_t launch_mover_f64(const MoverParams& m, bool ti, int fx, int ndim, int
     return launch_mover<PolicyF64>(m, ti, fx, ndim, 1, grid, s);
 }
 
-hipError_t launch_step_once_f64(const MoverParams& m, bool ti, int fx, int ndim, double* state,
-                                const double* rands, const int8_t* fixed, double* deltas,
+hipError_t launch_step_once_f64(const MoverParams& m, bool ti, int fx, int ndim, const StepRows& r,
                                 hipStream_t s) {
-    return launch_step_once<PolicyF64>(m, ti, fx, ndim, state, rands, fixed, deltas, s);
+    return launch_step_once<PolicyF64>(m, ti, fx, ndim, r, s);
 }
 
 hipError_t launch_order_digit_f64(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit, hipStream_t s) {

@@ -401,25 +401,64 @@ mover_kernel(MoverParams m0) {
     if (lane == 0 && my_paused) atomicAdd(&m.ctr->paused, my_paused);
 }
 
-// Single-step kernel for parity checks: caller-supplied states and increments.
+// Single-step kernel: caller-supplied states and increments, rows of 6 and 4
+// doubles, 64 rows per block, blockIdx.y the piece.  The rows pass through LDS so that each block
+// reads and writes them in 16-byte pieces in order, once: they may lie in
+// pinned host memory, where every piece is a transfer over PCIe.
+constexpr int kStepRows = 64;
 template <class Pol, int NDIM, bool TINTERP, int FX>
-__global__ void __launch_bounds__(256) step_once_kernel(MoverParams m, double* state,
-                                                        const double* rands, const int8_t* fixed,
-                                                        double* deltas) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m.n) return;
-    State s{state[6 * i + 0], state[6 * i + 1], state[6 * i + 2],
-            state[6 * i + 3], state[6 * i + 4], state[6 * i + 5], 0.0};
-    if constexpr ((FX & FX_NLGC) != 0) s.mu = m.P.d(PD_MU)[i];
-    double d[4] = {0.0, 0.0, 0.0, 0.0};
-    Pol::template step_given<NDIM, TINTERP, FX>(m, Pol::var_of(m), s, fixed[i] != 0, rands + 4 * i, d);
-    state[6 * i + 0] = s.x;
-    state[6 * i + 1] = s.y;
-    state[6 * i + 2] = s.z;
-    state[6 * i + 3] = s.p;
-    state[6 * i + 4] = s.t;
-    state[6 * i + 5] = s.dt;
-    for (int c = 0; c < 4; ++c) deltas[4 * i + c] = d[c];
+__global__ void __launch_bounds__(kStepRows) step_once_kernel(MoverParams m, StepRows sr) {
+    __shared__ double2 st2[kStepRows * 3], rd2[kStepRows * 2];
+    double* const st = reinterpret_cast<double*>(st2);
+    double* const rd = reinterpret_cast<double*>(rd2);
+    const long long i0 = (long long)blockIdx.x * kStepRows, i = i0 + threadIdx.x;
+    const int pc = blockIdx.y;
+    const long long left = sr.n[pc] - i0;
+    if (left <= 0) return;
+    const int rows = (int)(left < kStepRows ? left : kStepRows);
+    double2* const gs = reinterpret_cast<double2*>(sr.state[pc] + 6 * i0);
+    double2* const gd = reinterpret_cast<double2*>(sr.deltas[pc] + 4 * i0);
+    const double2* const gr = reinterpret_cast<const double2*>(sr.rands[pc] + 4 * i0);
+    const bool on = (int)threadIdx.x < rows;
+    const int8_t fx = on ? sr.fixed[pc][i] : (int8_t)0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int q = k * kStepRows + threadIdx.x;
+        if (q < 3 * rows) st2[q] = gs[q];
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int q = k * kStepRows + threadIdx.x;
+        if (q < 2 * rows) rd2[q] = gr[q];
+    }
+    __syncthreads();
+    if (on) {
+        double* const row = st + 6 * threadIdx.x;
+        double* const r = rd + 4 * threadIdx.x;
+        State s{row[0], row[1], row[2], row[3], row[4], row[5], 0.0};
+        if constexpr ((FX & FX_NLGC) != 0) s.mu = m.P.d(PD_MU)[sr.row0[pc] + i];
+        double d[4] = {0.0, 0.0, 0.0, 0.0};
+        const double rr[4] = {r[0], r[1], r[2], r[3]};
+        Pol::template step_given<NDIM, TINTERP, FX>(m, Pol::var_of(m), s, fx != 0, rr, d);
+        row[0] = s.x;
+        row[1] = s.y;
+        row[2] = s.z;
+        row[3] = s.p;
+        row[4] = s.t;
+        row[5] = s.dt;
+        for (int c = 0; c < 4; ++c) r[c] = d[c];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int q = k * kStepRows + threadIdx.x;
+        if (q < 3 * rows) gs[q] = st2[q];
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int q = k * kStepRows + threadIdx.x;
+        if (q < 2 * rows) gd[q] = rd2[q];
+    }
 }
 
 // Part of each particle (m.part_len) and the class of the step count that its
@@ -557,15 +596,16 @@ hipError_t launch_order_digit(const MoverParams& m, bool ti, int fx, int ndim, u
 }
 
 template <class Pol>
-hipError_t launch_step_once(const MoverParams& m, bool ti, int fx, int ndim, double* state,
-                            const double* rands, const int8_t* fixed, double* deltas,
+hipError_t launch_step_once(const MoverParams& m, bool ti, int fx, int ndim, const StepRows& r,
                             hipStream_t st) {
-    if (m.n <= 0) return hipSuccess;
-    const int grid = (int)((m.n + 255) / 256);
+    long long n = 0;
+    for (int k = 0; k < r.pieces; ++k) n = r.n[k] > n ? r.n[k] : n;
+    if (n <= 0) return hipSuccess;
+    const unsigned grid = (unsigned)((n + kStepRows - 1) / kStepRows);
     dispatch_variant<Pol>(ndim, ti, fx, [&](auto v) {
         using V = decltype(v);
-        hipLaunchKernelGGL((step_once_kernel<Pol, V::ndim, V::ti, V::fx>), dim3(grid), dim3(256),
-                           0, st, m, state, rands, fixed, deltas);
+        hipLaunchKernelGGL((step_once_kernel<Pol, V::ndim, V::ti, V::fx>), dim3(grid, (unsigned)r.pieces),
+                           dim3(kStepRows), 0, st, m, r);
         return 0;
     });
     return hipGetLastError();

@@ -98,6 +98,14 @@ hipError_t launch_dist(const Ptl& P, long long n, const DistArgs& da, unsigned l
 hipError_t launch_variant_dist(const Ptl& P, long long n, const DistArgs& da, int nvar,
                                unsigned long long* hist, unsigned long long* counts, int ncu,
                                hipStream_t s);
+// dst[k][i] = src[k][i] / kFxScale for up to kStagePieces pieces
+struct BinPieces {
+    const unsigned long long* src[kStagePieces];
+    double* dst[kStagePieces];
+    int n[kStagePieces];
+    int pieces;
+};
+hipError_t launch_bins_out(const BinPieces& b, hipStream_t s);
 hipError_t launch_stats(const Ptl& P, long long n, double* part, int grid, hipStream_t s);
 
 }  // namespace sp

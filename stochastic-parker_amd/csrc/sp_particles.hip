@@ -816,6 +816,26 @@ hipError_t launch_variant_dist(const Ptl& P, long long n, const DistArgs& da, in
     return hipGetLastError();
 }
 
+// Histogram bins as weights, into pinned host memory: bound by PCIe (1 MiB
+// in 22 us), which 64 blocks' 16-byte stores fill.  Written by a kernel, not
+// copied, so that the bins arrive as doubles and in one launch.
+__global__ void __launch_bounds__(kBlock) bins_out_kernel(BinPieces b) {
+    const int k = blockIdx.y, n2 = b.n[k] / 2;
+    const ulonglong2* const src = reinterpret_cast<const ulonglong2*>(b.src[k]);
+    double2* const dst = reinterpret_cast<double2*>(b.dst[k]);
+    const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    for (int i = t; i < n2; i += (int)(gridDim.x * blockDim.x)) {
+        const ulonglong2 v = src[i];
+        dst[i] = make_double2((double)v.x * (1.0 / kFxScale), (double)v.y * (1.0 / kFxScale));
+    }
+    if ((b.n[k] & 1) && t == 0) b.dst[k][b.n[k] - 1] = (double)b.src[k][b.n[k] - 1] * (1.0 / kFxScale);
+}
+
+hipError_t launch_bins_out(const BinPieces& b, hipStream_t s) {
+    hipLaunchKernelGGL(bins_out_kernel, dim3(16, (unsigned)b.pieces), dim3(kBlock), 0, s, b);
+    return hipGetLastError();
+}
+
 hipError_t launch_stats(const Ptl& P, long long n, double* part, int grid, hipStream_t s) {
     hipLaunchKernelGGL(stats_kernel, dim3(grid), dim3(kBlock), 0, s, P, n, part);
     return hipGetLastError();

@@ -145,7 +145,7 @@ class ParkerPusher:
 
     def get_particles(self) -> dict:
         n = self.counts()["nptl_current"]
-        arrs = empty_particles(n)
+        arrs = {name: np.empty(n, dtype=dt) for name, dt in PARTICLE_FIELDS}
         s = _soa_struct(arrs)
         got = C.c_int64()
         self._call("sp_particles_download", C.byref(s), n, C.byref(got))
@@ -207,7 +207,7 @@ class ParkerPusher:
         r = np.ascontiguousarray(rands, dtype=np.float64)
         fx = np.ascontiguousarray(fixed, dtype=np.int8)
         n = st.shape[0]
-        d = np.zeros((n, 4), dtype=np.float64)
+        d = np.empty((n, 4), dtype=np.float64)
         self._call("sp_step_once_noalloc" if noalloc else "sp_step_once", n, float(t0), float(dtf),
                    dptr(st), dptr(r), fx.ctypes.data_as(C.POINTER(C.c_int8)), dptr(d))
         return st, d
@@ -238,13 +238,13 @@ class ParkerPusher:
     def calc_particle_distributions(self):
         """Returns (fglobal, [flocal1..4]); flocal arrays are Fortran-ordered
         (nmu, npbins, nrx, nry, nrz) reshaped to C order (nrz, nry, nrx, npbins, nmu)."""
-        fg = np.zeros(self._npp, dtype=np.float64)
+        fg = np.empty(self._npp, dtype=np.float64)
         outs = []
         ptrs = []
         for d in self._dist_dims:
             size = int(np.prod(d)) if d[0] else 0
             if size:
-                a = np.zeros(size, dtype=np.float64)
+                a = np.empty(size, dtype=np.float64)
                 outs.append(a)
                 ptrs.append(dptr(a))
             else:

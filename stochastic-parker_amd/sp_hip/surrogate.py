@@ -73,7 +73,7 @@ class Mlp:
 
     def forward(self, x) -> np.ndarray:
         x = np.ascontiguousarray(x, dtype=np.float32).reshape(-1, self.shape[0])
-        y = np.zeros((len(x), self.shape[3]), dtype=np.float32)
+        y = np.empty((len(x), self.shape[3]), dtype=np.float32)
         self._call("sp_mlp_forward", self._f(x), len(x), self._f(y))
         return y
 
@@ -248,8 +248,8 @@ class Surrogate:
         both computed on the GPU."""
         x = np.ascontiguousarray(x, dtype=np.float32)
         n = len(x)
-        spec = np.zeros((n, self.nets[0].shape[3]), dtype=np.float32)
-        spread = np.zeros(n, dtype=np.float32)
+        spec = np.empty((n, self.nets[0].shape[3]), dtype=np.float32)
+        spread = np.empty(n, dtype=np.float32)
         hs = (C.c_void_p * len(self.nets))(*[m.h for m in self.nets])
         lib = self.nets[0].lib
         f = Mlp._f
