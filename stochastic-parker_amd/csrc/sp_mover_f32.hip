@@ -25,10 +25,10 @@ struct PolicyF32Base {
     using Cache = f32::GatherCache<NDIM, TI, HALF, (FX & FX_DPP) != 0, PPL>;
     template <int NDIM, bool TI, int FX, class GC>
     __device__ __forceinline__ static void step(const MoverParams& m, const Var& kf, State& s,
-                                                bool fixed, uint32_t tagi, uint32_t tags,
-                                                uint32_t rstep, double d[4], GC& gc) {
+                                                bool fixed, const PhiloxPtl& rng, uint32_t rstep,
+                                                double d[4], GC& gc) {
         float r[4];
-        f32::step_rands(m, tagi, tags, rstep, r);
+        f32::step_rands(m, rng, rstep, r);
         f32::gather_kappa_push<NDIM, TI, FX, HALF>(m, kf, s, fixed, r, d, gc);
     }
     // PPL particles: the Philox blocks, the gathers and the steps of all
@@ -39,7 +39,7 @@ struct PolicyF32Base {
                                                   double (*d)[4]) {
         float r[PPL][4];
 #pragma unroll
-        for (int k = 0; k < PPL; ++k) f32::step_rands(m, sl[k].tagi, sl[k].tags, sl[k].rstep, r[k]);
+        for (int k = 0; k < PPL; ++k) f32::step_rands(m, sl[k].rng, sl[k].rstep, r[k]);
         Cache<NDIM, TI, FX, PPL> none;   // no records kept across steps at PPL > 1
 #pragma unroll
         for (int k = 0; k < PPL; ++k)

@@ -26,10 +26,10 @@ struct PolicyF64 {
     using Cache = f64::CellCache<NDIM == 3 && !TI && (FX & FX_DPP) == 0>;
     template <int NDIM, bool TI, int FX, class GC>
     __device__ __forceinline__ static void step(const MoverParams& m, const Var&, State& s,
-                                                bool fixed, uint32_t tagi, uint32_t tags,
-                                                uint32_t rstep, double d[4], GC& gc) {
+                                                bool fixed, const PhiloxPtl& rng, uint32_t rstep,
+                                                double d[4], GC& gc) {
         double r[4];
-        f64::step_rands(m, tagi, tags, rstep, r);
+        f64::step_rands(m, rng, rstep, r);
         f64::gather_kappa_push<NDIM, TI, FX>(m, s, fixed, r, d, gc);
     }
     template <int NDIM, bool TI, int FX>

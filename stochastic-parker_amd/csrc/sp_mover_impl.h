@@ -77,7 +77,8 @@ struct Slot {
     double w, dtarget, dt_old;
     double dl[4];                 // the last step's increments (for the undo)
     int cf, nsp, pending;
-    uint32_t tagi, tags, rstep;
+    PhiloxPtl rng;
+    uint32_t rstep;
     unsigned ksteps;              // steps of this particle in this launch
     bool resumed;
 };
@@ -155,7 +156,8 @@ mover_kernel(MoverParams m0) {
         sl[k].dl[0] = sl[k].dl[1] = sl[k].dl[2] = sl[k].dl[3] = 0.0;
         sl[k].cf = sl[k].nsp = 0;
         sl[k].pending = PEND_NONE;
-        sl[k].tagi = sl[k].tags = sl[k].rstep = 0u;
+        sl[k].rng = PhiloxPtl{0u, 0u, 0u, 0u};
+        sl[k].rstep = 0u;
         sl[k].ksteps = 0u;
         sl[k].resumed = false;
         var[k] = Pol::var_of(m);
@@ -168,7 +170,7 @@ mover_kernel(MoverParams m0) {
         for (int k = 0; k < PPL; ++k) {
             Slot& q = sl[k];
             const bool need = q.idx < 0 && !exhausted;
-            const unsigned long long need_mask = __ballot(need);
+            const unsigned long long need_mask = __builtin_amdgcn_ballot_w64(need);
             if (!need_mask) continue;
             const int leader = __ffsll((unsigned long long)need_mask) - 1;
             const unsigned long long cnt = (unsigned long long)__popcll(need_mask);
@@ -205,8 +207,8 @@ mover_kernel(MoverParams m0) {
                         v = v < 0 ? 0 : (v >= m0.nvar ? m0.nvar - 1 : v);
                         Pol::set_var(m, var[k], m0.var[v]);
                     }
-                    q.tagi = (uint32_t)m.P.i(PI_TAGI)[j];
-                    q.tags = (uint32_t)m.P.i(PI_TAGS)[j];
+                    q.rng = philox_ptl((uint32_t)m.P.i(PI_TAGI)[j], (uint32_t)m.P.i(PI_TAGS)[j], m.stream,
+                                       m.key0, m.key1);
                     q.rstep = prstep[j];
                     q.dl[0] = q.dl[1] = q.dl[2] = q.dl[3] = 0.0;
                     q.ksteps = 0;
@@ -229,7 +231,7 @@ mover_kernel(MoverParams m0) {
         bool busy = false;
 #pragma unroll
         for (int k = 0; k < PPL; ++k) busy = busy || sl[k].idx >= 0;
-        if (__ballot(busy || !exhausted) == 0ull) break;
+        if (__builtin_amdgcn_ballot_w64(busy || !exhausted) == 0ull) break;
 
         bool do_push[PPL], fixed[PPL];
 #pragma unroll
@@ -315,6 +317,7 @@ mover_kernel(MoverParams m0) {
             } else if (act == ACT_PUSH_FIXED) {
                 do_push[k] = true;
                 fixed[k] = true;
+                q.pending = PEND_REDO;
             } else if (act == ACT_ADVANCE) {
                 q.dtarget = q.dtarget + m.dt_fine;
                 fin = !(q.dtarget < m.dt_limit) || q.cf != SP_COUNT_FLAG_INBOX;
@@ -345,6 +348,7 @@ mover_kernel(MoverParams m0) {
                 pflag[j] = (int8_t)q.cf;
                 ppushed[j] = q.nsp;
                 prstep[j] = q.rstep;
+                my_steps += q.ksteps;
                 q.idx = -1;
             }
         }
@@ -355,8 +359,8 @@ mover_kernel(MoverParams m0) {
         for (int k = 0; k < PPL; ++k) any_push = any_push || do_push[k];
         if (any_push) {
             if constexpr (PPL == 1) {
-                Pol::template step<NDIM, TINTERP, FX>(m, var[0], sl[0].s, fixed[0], sl[0].tagi,
-                                                      sl[0].tags, sl[0].rstep, sl[0].dl, gc);
+                Pol::template step<NDIM, TINTERP, FX>(m, var[0], sl[0].s, fixed[0], sl[0].rng,
+                                                      sl[0].rstep, sl[0].dl, gc);
             } else {
                 // every slot steps (one straight-line block); a slot without a
                 // step to take keeps its state
@@ -384,9 +388,7 @@ mover_kernel(MoverParams m0) {
                 int v = q.nsp + 1;  // mod(nsteps_pushed + 1, nsteps_interval)
                 if ((unsigned)v >= (unsigned)m.nsteps_interval) v %= m.nsteps_interval;
                 q.nsp = v;
-                ++my_steps;
                 ++q.ksteps;
-                if (fixed[k]) q.pending = PEND_REDO;
             }
         }
     }

@@ -52,15 +52,15 @@ __device__ __forceinline__ Interp interp_params(const MoverParams& m, double x, 
     const double py = (y - m.ymin) * m.idy;
     const double fx = floor(px), fy = floor(py);
     const float rx = (float)(px - fx), ry = (float)(py - fy);
-    I.ix = clamp_cell(fx, m.nxg - 4) + 2;
-    I.iy = clamp_cell(fy, m.nyg - 4) + 2;
+    I.ix = step_cell(fx, m.nxg - 4) + 2;
+    I.iy = step_cell(fy, m.nyg - 4) + 2;
     I.iz = 0;
     float rz = 0.0f;
     if (NDIM == 3) {
         const double pz = (z - m.zmin) * m.idz;
         const double fz = floor(pz);
         rz = (float)(pz - fz);
-        I.iz = clamp_cell(fz, m.nzg - 4) + 2;
+        I.iz = step_cell(fz, m.nzg - 4) + 2;
     }
     I.rx = rx;
     I.ry = ry;
@@ -593,7 +593,7 @@ __device__ __forceinline__ void kappa_push(const MoverParams& m, const KF& kf, S
         dx_dt = f[R2_VX] + vdx + dkxx_dx + dkxy_dy;
         dy_dt = f[R2_VY] + vdy + dkxy_dx + dkyy_dy;
         dz_dt = vdz;
-        divv = f[R2_DVXDX] + f[R2_DVYDY];
+        divv = DPP ? f[R2_DVXDX] + f[R2_DVYDY] : f[R2_DVXDX];   // the compact records hold div V there
     } else {
         const float dbx_dx = f[R3_DBXDX], dbx_dy = f[R3_DBXDY], dbx_dz = f[R3_DBXDZ];
         const float dby_dx = f[R3_DBYDX], dby_dy = f[R3_DBYDY], dby_dz = f[R3_DBYDZ];
@@ -653,7 +653,7 @@ __device__ __forceinline__ void kappa_push(const MoverParams& m, const KF& kf, S
         dx_dt = f[R3_VX] + vdx + dkxx_dx + dkxy_dy + dkxz_dz;
         dy_dt = f[R3_VY] + vdy + dkxy_dx + dkyy_dy + dkyz_dz;
         dz_dt = f[R3_VZ] + vdz + dkxz_dx + dkyz_dy + dkzz_dz;
-        divv = f[R3_DVXDX] + f[R3_DVYDY] + f[R3_DVZDZ];
+        divv = DPP ? f[R3_DVXDX] + f[R3_DVYDY] + f[R3_DVZDZ] : f[R3_DVXDX];
     }
     float dp_dt = -pf * divv * (1.0f / 3.0f);
     float dpp = 0.0f;
@@ -672,8 +672,7 @@ __device__ __forceinline__ void kappa_push(const MoverParams& m, const KF& kf, S
     if (NDIM == 3) { a = sk * frcp(dz_dt); mm = fminf(mm, a * a); }
     mm = fminf(mm, 0.1f * pf * frcp(fabsf(dp_dt)));
     const bool rates = dx_dt != 0.0f && dy_dt != 0.0f && dp_dt != 0.0f;
-    mm = rates ? mm : m.f_dt_min;
-    mm = fminf(fmaxf(mm, m.f_dt_min), m.f_dt_max);
+    mm = __builtin_amdgcn_fmed3f(rates ? mm : 0.0f, m.f_dt_min, m.f_dt_max);   // 0 < dt_min <= dt_max
     s.dt = fixed_dt ? s.dt : (double)mm;
     const float dtf32 = fixed_dt ? (float)s.dt : mm;
     const float sdt = fsqrt(dtf32);
@@ -708,11 +707,14 @@ __device__ __forceinline__ void kappa_push(const MoverParams& m, const KF& kf, S
     } else {
         s.p += dp;
     }
-    // momentum floor: back out the increment, land on 0.25 p0
+    // momentum floor: back out the increment, land on 0.25 p0.  Rare: a wave
+    // without such a particle skips the two differences and the selects.
     const bool low = s.p < m.p_floor;
-    const double pback = s.p - dp;
-    dp = low ? m.p_floor - pback : dp;
-    s.p = low ? m.p_floor : s.p;
+    if (__builtin_amdgcn_ballot_w64(low)) {
+        const double pback = s.p - dp;
+        dp = low ? m.p_floor - pback : dp;
+        s.p = low ? m.p_floor : s.p;
+    }
     d[0] = (double)deltax;
     d[1] = (double)deltay;
     d[2] = NDIM == 2 ? 0.0 : (double)deltaz;
@@ -720,9 +722,9 @@ __device__ __forceinline__ void kappa_push(const MoverParams& m, const KF& kf, S
 }
 
 // (2u - 1) sqrt(3) in FP32 from one Philox block: u = r / (2^32 - 1).
-__device__ __forceinline__ void step_rands(const MoverParams& m, uint32_t tag_i, uint32_t tag_s,
-                                           uint32_t step, float r[4]) {
-    const U4 u = philox4x32_10(tag_i, tag_s, step, m.stream, m.key0, m.key1);
+__device__ __forceinline__ void step_rands(const MoverParams& m, const PhiloxPtl& rng, uint32_t step,
+                                           float r[4]) {
+    const U4 u = philox_step(rng, step, m.key0, m.key1);
     const float sc = (float)(2.0 * 1.7320508075688772 / 4294967295.0);
     const float of = -1.7320508075688772f;
     r[0] = (float)u.a * sc + of;

@@ -46,14 +46,14 @@ __device__ __forceinline__ Interp interp_params(const MoverParams& m, double x, 
     const double rx = (px - (fx + 1.0)) + 1.0;  // px - pos + 1 with pos = floor(px) + 1
     const double ry = (py - (fy + 1.0)) + 1.0;
     double rz = 0.0;
-    I.ix = clamp_cell(fx, m.nxg - 4) + 2;
-    I.iy = clamp_cell(fy, m.nyg - 4) + 2;
+    I.ix = step_cell(fx, m.nxg - 4) + 2;
+    I.iy = step_cell(fy, m.nyg - 4) + 2;
     I.iz = 0;
     if (NDIM == 3) {
         const double pz = div_const(z - m.zmin, m.dz, m.idz);
         const double fz = floor(pz);
         rz = (pz - (fz + 1.0)) + 1.0;
-        I.iz = clamp_cell(fz, m.nzg - 4) + 2;
+        I.iz = step_cell(fz, m.nzg - 4) + 2;
     }
     const double rx1 = 1.0 - rx, ry1 = 1.0 - ry, rz1 = 1.0 - rz;
     I.w[0] = rx1 * ry1 * rz1;
@@ -542,9 +542,9 @@ __device__ __forceinline__ void push(const MoverParams& m, State& s, const doubl
 
 // Steps' increments from one Philox block: (2u - 1) * sqrt(3) for each
 // of the four words (particle_module.f90:3548-3550, :3589).
-__device__ __forceinline__ void step_rands(const MoverParams& m, uint32_t tag_i, uint32_t tag_s,
-                                           uint32_t step, double r[4]) {
-    const U4 u = philox4x32_10(tag_i, tag_s, step, m.stream, m.key0, m.key1);
+__device__ __forceinline__ void step_rands(const MoverParams& m, const PhiloxPtl& rng, uint32_t step,
+                                           double r[4]) {
+    const U4 u = philox_step(rng, step, m.key0, m.key1);
     const double sqrt3 = sqrt(3.0);
     r[0] = (2.0 * u01(u.a) - 1.0) * sqrt3;
     r[1] = (2.0 * u01(u.b) - 1.0) * sqrt3;
