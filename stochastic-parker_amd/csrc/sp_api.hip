@@ -987,15 +987,20 @@ int mover_run(Ctx* c, double t0, double dtf, int num_fine_steps, int nsteps_inte
         // handed out in spatial order, a long one that starts last runs on alone.
         // So the parts hand out those with the smaller first step first: 64
         // variants, 1.2e6 particles on 512^2, 6.9 -> 5.0 ms (two intervals'
-        // mean, FP32; FP64 14.2 -> 10.7).  Only from 1 to 16 particles per lane:
-        // with fewer nothing waits for a lane; at 16 the order still gains 9 %,
-        // at 44 it loses 3 % (the classes' sparser windows of the sorted
-        // particles share fewer records, and the tail is short).  Not for
-        // single-variant runs: their steps differ little at the start, and in
-        // 3D turbulence the first step does not tell (5-10 % slower).
+        // mean, FP32; FP64 14.2 -> 10.7).  Not below one particle per lane
+        // (nothing waits for a lane), and not for single-variant runs: their
+        // steps differ little at the start, and in 3D turbulence the first step
+        // does not tell (5-10 % slower).  The FP32 kernel's lanes wait for the
+        // wave's other work (MF_WAIT) from 5 particles per lane up: 3.3 a lane
+        // 15 % slower, 6 a lane 8 % faster, 19 a lane 14 %, 80 a lane 62.5 ->
+        // 54.4 ms.  Without that the order gains up to 16 a lane (9 %) and loses
+        // 3 % at 44: the classes' sparser windows of the sorted particles share
+        // fewer records, and the tail is short.
         const long long lanes = 256ll * ppl * grid;
+        const bool wait = c->cfg.precision == SP_PREC_F32 && nrun > 5 * lanes;
         const bool ordered = c->nvar > 1 && c->cfg.ndim == 2 && !ti && (fx & ~sp::FX_LEAN) == 0 && ppl == 1 &&
-                             m.step_budget == 0u && nrun > lanes && nrun <= 16 * lanes;
+                             m.step_budget == 0u && nrun > lanes && (wait || nrun <= 16 * lanes);
+        if (ordered && wait) m.flags |= sp::MF_WAIT;
         if (ordered) {
             rc = sort_buffers(c);
             if (rc != SP_OK) return rc;

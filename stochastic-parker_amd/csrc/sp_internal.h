@@ -195,7 +195,8 @@ struct KappaVar {
 enum MoverFlags {
     MF_OPEN_X = 1, MF_OPEN_Y = 2, MF_OPEN_Z = 4,
     MF_MOMENTUM_DEP = 8, MF_MAG_DEP = 16, MF_DRIFT_2D = 32,
-    MF_DPP_WAVE = 64, MF_DPP_SHEAR = 128, MF_WEAK_SCATTERING = 256
+    MF_DPP_WAVE = 64, MF_DPP_SHEAR = 128, MF_WEAK_SCATTERING = 256,
+    MF_WAIT = 512   // with order: the kernel whose lanes wait (kServeLanes)
 };
 
 // Kernel arguments of the mover and of the single-step kernel: only the

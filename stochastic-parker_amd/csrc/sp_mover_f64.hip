@@ -9,6 +9,7 @@ namespace sp {
 // overwrite the lane's own copy of the kernel arguments when it takes a
 // particle, so Var carries nothing.
 struct PolicyF64 {
+    static constexpr bool kWaits = false;   // no gain
     static constexpr bool kOnly3D = false;
     static constexpr bool kDpp = true;
     static constexpr int kMaxPPL = 1;

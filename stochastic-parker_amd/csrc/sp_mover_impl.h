@@ -109,12 +109,23 @@ constexpr bool kThreeWave = Pol::kThreeWave2D && NDIM == 2 && !TINTERP && PPL ==
 
 // ORDER: the parts hand out particles in the order of m.order (a kernel of its
 // own: the test and the pointer in the other kernels cost them 2-3 %).
-template <class Pol, int NDIM, bool TINTERP, int FX, int PPL, bool ORDER = false>
+// WAIT: the wave's other work (taking a particle, landing on a target time,
+// leaving) comes to one lane in most iterations and costs the whole wave its
+// instructions.  So these lanes wait until together they have lost kServeLanes
+// iterations, or are an eighth of the lanes that step (64 variants, 3.8e6
+// particles on 512^2, two intervals: at once 25.4 ms, 2 lane-iterations 23.5, 4
+// 22.7, 8 22.0, 16 21.6).  A kernel of its own, for lanes that take many
+// particles in turn: where they take a few, the last ones' chains of steps are
+// drawn out (-15 %), and the votes alone cost 5 %.
+constexpr int kServeLanes = 16;
+template <class Pol, int NDIM, bool TINTERP, int FX, int PPL, bool ORDER = false, bool WAIT = false>
 __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(kThreeWave<Pol, NDIM, TINTERP, PPL> ? 3 : (kTwoWavePair<NDIM, PPL> ? 2 : 1),
                                    kThreeWave<Pol, NDIM, TINTERP, PPL> ? 3 : 2)))
 mover_kernel(MoverParams m0) {
     static_assert(PPL >= 1 && PPL <= Pol::kMaxPPL, "particles per lane of this policy");
+    constexpr int kServe = WAIT ? kServeLanes : 0;
+    static_assert(!WAIT || PPL == 1, "one slot waits");
     MoverParams m = m0;
     // within the two-wave register budget the constants fit in VGPRs for 2D
     // and 3D alike (2D: +5 %, 3D: +1 %)
@@ -163,11 +174,14 @@ mover_kernel(MoverParams m0) {
         var[k] = Pol::var_of(m);
     }
     unsigned long long my_steps = 0, my_paused = 0;
+    bool serve = true;            // this iteration does the wave's other work (kServeLanes)
+    int waited = 0;               // lane-iterations lost since it was last done
 
     while (true) {
         // ---- refill idle slots (wave-aggregated work fetch, one slot index at a time) ----
 #pragma unroll
         for (int k = 0; k < PPL; ++k) {
+            if (kServe > 0 && !serve) break;
             Slot& q = sl[k];
             const bool need = q.idx < 0 && !exhausted;
             const unsigned long long need_mask = __builtin_amdgcn_ballot_w64(need);
@@ -257,6 +271,7 @@ mover_kernel(MoverParams m0) {
                     continue;
                 }
             }
+            if (kServe > 0 && !serve) continue;
             // ---- choose this slot's action ----
             int act = ACT_NONE;
             bool need_bc = false;
@@ -350,6 +365,18 @@ mover_kernel(MoverParams m0) {
                 prstep[j] = q.rstep;
                 my_steps += q.ksteps;
                 q.idx = -1;
+            }
+        }
+
+        if constexpr (kServe > 0) {
+            const unsigned long long wm = __builtin_amdgcn_ballot_w64(sl[0].idx >= 0 ? !do_push[0] : !exhausted);
+            const unsigned long long pm = __builtin_amdgcn_ballot_w64(do_push[0]);
+            if (serve) {
+                waited = 0;
+                serve = pm == 0ull;
+            } else {
+                waited += __popcll(wm);
+                serve = waited >= kServe || __popcll(wm) * 8 >= __popcll(pm);
             }
         }
 
@@ -569,10 +596,19 @@ hipError_t launch_mover(const MoverParams& m, bool ti, int fx, int ndim, int ppl
             using V = decltype(vv);
             constexpr int kPpl = decltype(pc)::value;
             if (m.order) {
-                if constexpr (kOrdered<V> && kPpl == 1)
+                if constexpr (kOrdered<V> && kPpl == 1) {
+                    if constexpr (Pol::kWaits) {
+                        if (m.flags & MF_WAIT) {
+                            hipLaunchKernelGGL((mover_kernel<Pol, V::ndim, V::ti, V::fx, 1, true, true>),
+                                               dim3(grid), dim3(256), 0, st, m);
+                            return 1;
+                        }
+                    }
                     hipLaunchKernelGGL((mover_kernel<Pol, V::ndim, V::ti, V::fx, 1, true>), dim3(grid),
                                        dim3(256), 0, st, m);
-                return kOrdered<V> && kPpl == 1 ? 1 : 0;
+                    return 1;
+                }
+                return 0;
             }
             hipLaunchKernelGGL((mover_kernel<Pol, V::ndim, V::ti, V::fx, kPpl>), dim3(grid), dim3(256), 0, st,
                                m);
