@@ -10,7 +10,10 @@
 // and every back-propagated pre-activation gradient; all products accumulate
 // in FP32.
 //
-// GEMM (training): 128 x 128, 128 x 64 or 64 x 64 output tiles per 256-lane
+// Training steps of the usual shapes are two launches (sp_mlp_train.h), small
+// queries one (sp_mlp_query.h).
+//
+// GEMM (training of the other shapes): 128 x 128, 128 x 64 or 64 x 64 output tiles per 256-lane
 // block, four waves of a quarter tile each, K in steps of 32 staged through LDS
 // as k-contiguous BF16 rows with 16-byte loads, v_mfma_f32_32x32x16_bf16 on the
 // wave's 32 x 32 tiles.  Inference of the usual shapes runs all layers in one
