@@ -13,6 +13,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -31,6 +32,9 @@ int fail(int code, const std::string& msg) {
 }  // namespace
 
 int sp::set_error(int code, const std::string& msg) { return fail(code, msg); }
+
+int sp::PinnedMem::get(void** p, size_t bytes) { return (int)hipHostMalloc(p, bytes, hipHostMallocDefault); }
+void sp::PinnedMem::drop(void* p) { (void)hipHostFree(p); }
 
 namespace {
 
@@ -53,15 +57,10 @@ constexpr int kMoverBlocksPerCU3D = 1;
 // Particles per lane of the FP32 movers unless tuned or overridden.
 constexpr int kMoverPPLDefault = 1;
 
-// Pinned host staging of a context: Ctx::pin for counters and partial sums,
-// and two groups of sp::kStagePieces slots for histograms and for the rows of
-// sp_step_once (a row: state, deltas, random numbers, flag).  256 KiB a slot,
-// each allocated when first used: pinned allocations of up to that size cost
-// 14 us, larger ones 0.3 ms and as much again for the first touch of their pages.
-constexpr int kPinSlots = 2 * sp::kStagePieces;
-constexpr size_t kPinSmall = 64 << 10, kPinSlot = 256 << 10;
-constexpr long long kSlotRows = 2304, kSlotBins = kPinSlot / sizeof(double);
-static_assert(kSlotRows % 64 == 0 && kSlotRows * (14 * sizeof(double) + 1) <= kPinSlot, "rows fit a slot");
+// Pinned slots hold a call's counters and partial sums (PinResults), its
+// histograms, or its rows of sp_step_once (state, deltas, random numbers, flag).
+constexpr long long kSlotRows = 2304, kSlotBins = sp::kSlotBytes / sizeof(double);
+static_assert(kSlotRows % 64 == 0 && kSlotRows * (14 * sizeof(double) + 1) <= sp::kSlotBytes, "rows fit a slot");
 
 struct Ctx {
     sp_config cfg{};
@@ -97,9 +96,7 @@ struct Ctx {
     long long mover_calls = 0;
     // autotuned launch settings (0 / -1: not tuned) and the tuner's state copy
     int tuned_bpc = 0, tuned_sort_steps = -1;
-    void* pin = nullptr;                   // kPinSmall
-    void* slot[kPinSlots] = {};            // kPinSlot each
-    hipEvent_t slot_ev[2] = {};            // the groups' last kernels
+    hipEvent_t slot_ev[2] = {};            // last kernels of the two groups of pieces
     void* pbuf_save = nullptr;
     // batched parameter variants
     sp::KappaVar* dvar = nullptr;
@@ -141,6 +138,19 @@ static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 void* g_scratch[kMaxDevices] = {};
+
+// One pool of pinned slots per GPU for the life of the process (never torn
+// down: the HIP runtime may end before static objects do).  It keeps up to 8 MiB.
+using PinnedPool = sp::SlotPool<sp::PinnedMem, 32>;
+std::mutex g_pool_mu;
+PinnedPool* g_pool[kMaxDevices] = {};
+
+PinnedPool* pinned_pool(int device) {
+    if (device < 0 || device >= kMaxDevices) return nullptr;
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    if (!g_pool[device]) g_pool[device] = new (std::nothrow) PinnedPool;
+    return g_pool[device];
+}
 
 // Looks up this GPU's copy of `scratch` once (the device must be current).
 int init_scratch(int device) {
@@ -318,45 +328,39 @@ int mover_grid(Ctx* c, long long n, int bpc = 0, int ppl = 1) {
     return (int)std::max<long long>(1, std::min(need, cap));
 }
 
-// Pinned results of one call, in c->pin's small part: quick_check partials,
-// counters, removal totals.
+// Pinned results of one call, in one slot: quick_check partials, counters,
+// removal totals.
 struct PinResults {
     double stats[5 * 1024];      // stats_grid rows
     sp::Counters ctr;
     unsigned long long totals[2];
 };
-static_assert(sizeof(PinResults) <= kPinSmall, "fits the small part");
+static_assert(sizeof(PinResults) <= sp::kSlotBytes, "fits a slot");
 
-int pin_buffer(Ctx* c) {
-    if (!c->pin) SP_HIP(hipHostMalloc(&c->pin, kPinSmall, hipHostMallocDefault));
-    return SP_OK;
-}
-PinResults* pin_results(Ctx* c) { return reinterpret_cast<PinResults*>(c->pin); }
-
-// Sends `count` pieces through the slots, in groups of sp::kStagePieces:
+// Sends `count` pieces through pinned slots, in groups of sp::kStagePieces:
 // submit(first, pieces, slots) fills slots and launches the kernel that reads
 // or writes them, drain does what follows it on the host, while the other
-// group's kernel runs.  The stream is idle afterwards.
+// group's kernel runs.  The stream is idle afterwards.  The slots are taken
+// before anything is submitted: without memory for them nothing has happened.
 template <typename Submit, typename Drain>
 hipError_t pipe_pieces(Ctx* c, long long count, Submit submit, Drain drain) {
     constexpr int G = sp::kStagePieces;
     const long long groups = (count + G - 1) / G;
     auto pieces = [&](long long g) { return (int)std::min<long long>(G, count - g * G); };
-    hipError_t e = hipSuccess;
+    sp::PinnedSlots pin(c->device, c->st);
+    hipError_t e = pin.take((int)std::min<long long>(2 * G, count));
+    if (e != hipSuccess) return e;
     for (long long g = 0; g <= groups && e == hipSuccess; ++g) {
-        void** const slots = c->slot + (g & 1) * G;
         if (g < groups) {
-            for (int k = 0; k < pieces(g) && e == hipSuccess; ++k)
-                if (!slots[k]) e = hipHostMalloc(&slots[k], kPinSlot, hipHostMallocDefault);
-            if (e == hipSuccess) e = submit(g * G, pieces(g), slots);
+            e = submit(g * G, pieces(g), pin.slots() + (g & 1) * G);
             if (e == hipSuccess && g + 1 < groups) e = hipEventRecord(c->slot_ev[g & 1], c->st);
         }
         if (g > 0 && e == hipSuccess) {
             e = g < groups ? hipEventSynchronize(c->slot_ev[(g - 1) & 1]) : hipStreamSynchronize(c->st);
-            if (e == hipSuccess) drain((g - 1) * G, pieces(g - 1), c->slot + ((g - 1) & 1) * G);
+            if (e == hipSuccess) drain((g - 1) * G, pieces(g - 1), pin.slots() + ((g - 1) & 1) * G);
         }
     }
-    if (e != hipSuccess) (void)hipStreamSynchronize(c->st);   // nothing may write to the slots any more
+    pin.idle(e == hipSuccess);
     return e;
 }
 
@@ -580,9 +584,6 @@ void destroy(Ctx* c) {
     free_dev(c->vhist);
     free_dev(c->gmax);
     free_dev(c->pbuf_save);
-    if (c->pin) (void)hipHostFree(c->pin);
-    for (auto& p : c->slot)
-        if (p) (void)hipHostFree(p);
     for (auto& e : c->ev)
         if (e) (void)hipEventDestroy(e);
     for (auto& e : c->slot_ev)
@@ -592,6 +593,20 @@ void destroy(Ctx* c) {
 }
 
 }  // namespace
+
+hipError_t sp::PinnedSlots::take(int n) {
+    PinnedPool* const pool = pinned_pool(device_);
+    if (!pool || n > kMax) return hipErrorInvalidValue;
+    const hipError_t e = (hipError_t)pool->take(s_, n);
+    if (e == hipSuccess) n_ = n;
+    return e;
+}
+
+sp::PinnedSlots::~PinnedSlots() {
+    if (n_ == 0) return;
+    if (!idle_) (void)hipStreamSynchronize(st_);
+    pinned_pool(device_)->give(s_, n_);
+}
 
 extern "C" {
 
@@ -951,12 +966,12 @@ int sp_inject_particles_threshold(void* ctx, int32_t quantity, int64_t nptl, dou
 // bpc > 0 / sort_steps >= 0 override the launch settings (autotuner trials).
 // With `deferred`, the steps and the time of a last launch without a budget
 // are left to the caller, who reads them after its own next synchronisation.
+// Counters pass through pr.
 int mover_run(Ctx* c, double t0, double dtf, int num_fine_steps, int nsteps_interval, int bpc,
               int sort_steps, int ppl_trial, unsigned long long& steps, float& ms_push,
-              bool* deferred = nullptr) {
+              PinResults* pr, bool* deferred = nullptr) {
     const int ppl = mover_ppl(c, ppl_trial);
-    int rc = pin_buffer(c);
-    if (rc != SP_OK) return rc;
+    int rc = SP_OK;
     const bool ti = c->cfg.time_interp != 0;
     const int fx = step_features(c->cfg);
     // With sort_steps, the interval runs as launches of at most sort_steps
@@ -1022,7 +1037,7 @@ int mover_run(Ctx* c, double t0, double dtf, int num_fine_steps, int nsteps_inte
             *deferred = true;
             return SP_OK;
         }
-        sp::Counters* const hc = &pin_results(c)->ctr;
+        sp::Counters* const hc = &pr->ctr;
         SP_HIP(hipMemcpyAsync(&hc->steps, &c->ctr->steps, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, c->st));
         SP_HIP(hipStreamSynchronize(c->st));
         float ms = 0.f;
@@ -1048,6 +1063,9 @@ int sp_particle_mover(void* ctx, double t0, double dtf, int32_t num_fine_steps,
     if (c->cfg.time_interp && !c->have_fields[1]) return fail(SP_ERR_STATE, "time_interp needs slot 1 prepared");
     if (num_fine_steps < 1 || nsteps_interval < 1) return fail(SP_ERR_ARG, "num_fine_steps and nsteps_interval must be >= 1");
     if (!(dtf > 0)) return fail(SP_ERR_ARG, "dtf must be > 0");
+    sp::PinnedSlots pin(c->device, c->st);
+    SP_HIP(pin.take(1));
+    PinResults* const pr = static_cast<PinResults*>(pin.slots()[0]);
     const bool sorting = c->cfg.sort_every > 0;
     SP_HIP(hipEventRecord(c->ev[0], c->st));
     if (sorting && c->mover_calls % c->cfg.sort_every == 0) {
@@ -1058,7 +1076,7 @@ int sp_particle_mover(void* ctx, double t0, double dtf, int32_t num_fine_steps,
     unsigned long long steps = 0;
     float ms_push = 0.f;
     bool deferred = false;
-    rc = mover_run(c, t0, dtf, num_fine_steps, nsteps_interval, 0, -1, 0, steps, ms_push, &deferred);
+    rc = mover_run(c, t0, dtf, num_fine_steps, nsteps_interval, 0, -1, 0, steps, ms_push, pr, &deferred);
     if (rc != SP_OK) return rc;
     // remove_particles: stable compaction into the other buffer set
     long long kept = 0, esc = 0;
@@ -1071,13 +1089,13 @@ int sp_particle_mover(void* ctx, double t0, double dtf, int32_t num_fine_steps,
         SP_HIP(sp::launch_compact_scatter(c->P[c->cur], c->P[1 - c->cur], c->nptl, c->tile_off, c->st));
     }
     SP_HIP(hipEventRecord(c->ev[2], c->st));
-    PinResults* const pr = pin_results(c);
     SP_HIP(hipMemcpyAsync(&pr->ctr, c->ctr, sizeof(pr->ctr), hipMemcpyDeviceToHost, c->st));
     // the leak counters of this call move to the host totals (a u64 of 2^-32
     // units would wrap after a cumulative weight of 2^32)
     SP_HIP(hipMemsetAsync(&c->ctr->leak_fx, 0, 2 * sizeof(unsigned long long), c->st));
     if (c->nptl > 0) SP_HIP(hipMemcpyAsync(pr->totals, c->totals, sizeof(pr->totals), hipMemcpyDeviceToHost, c->st));
     SP_HIP(hipStreamSynchronize(c->st));
+    pin.idle(true);
     if (deferred) {
         float ms = 0.f;
         SP_HIP(hipEventElapsedTime(&ms, c->ev[1], c->ev[3]));
@@ -1396,6 +1414,9 @@ int sp_autotune_mover(void* ctx, double t0, double dtf, int32_t num_fine_steps,
     if (num_fine_steps < 1 || nsteps_interval < 1) return fail(SP_ERR_ARG, "num_fine_steps and nsteps_interval must be >= 1");
     if (!(dtf > 0)) return fail(SP_ERR_ARG, "dtf must be > 0");
     if (c->nptl < 1) return fail(SP_ERR_STATE, "no particles to tune on");
+    sp::PinnedSlots pin(c->device, c->st);
+    SP_HIP(pin.take(1));
+    PinResults* const pr = static_cast<PinResults*>(pin.slots()[0]);
     const long long cap = particle_cap(c->nmax);
     const size_t bytes = (size_t)sp::kPtlBytes * (size_t)cap;
     if (!c->pbuf_save) SP_HIP(hipMalloc(&c->pbuf_save, bytes));
@@ -1435,7 +1456,7 @@ int sp_autotune_mover(void* ctx, double t0, double dtf, int32_t num_fine_steps,
         }
         unsigned long long steps = 0;
         float ms = 0.f;
-        rc = mover_run(c, t0, dtf, num_fine_steps, nsteps_interval, tr.bpc, tr.ss, tr.ppl, steps, ms);
+        rc = mover_run(c, t0, dtf, num_fine_steps, nsteps_interval, tr.bpc, tr.ss, tr.ppl, steps, ms, pr);
         if (rc != SP_OK) break;
         const double rate = ms > 0.f ? (double)steps / (1e-3 * (double)ms) : 0.0;
         if (t < 0) {
@@ -1593,13 +1614,15 @@ int sp_quick_check(void* ctx, double out[9]) {
     if (!c) return rc;
     if (!out) return fail(SP_ERR_ARG, "out is NULL");
     const int grid = (int)std::max<long long>(1, std::min<long long>((c->nptl + 255) / 256, c->stats_grid));
-    if ((rc = pin_buffer(c)) != SP_OK) return rc;
-    PinResults* const pr = pin_results(c);
+    sp::PinnedSlots pin(c->device, c->st);
+    SP_HIP(pin.take(1));
+    PinResults* const pr = static_cast<PinResults*>(pin.slots()[0]);
     const double* const part = pr->stats;   // written by the kernel
     const sp::Counters& hc = pr->ctr;
     SP_HIP(sp::launch_stats(c->P[c->cur], c->nptl, pr->stats, grid, c->st));
     SP_HIP(hipMemcpyAsync(&pr->ctr, c->ctr, sizeof(pr->ctr), hipMemcpyDeviceToHost, c->st));
     SP_HIP(hipStreamSynchronize(c->st));
+    pin.idle(true);
     unsigned long long W = 0;
     double S = 0.0, mn = 1.0, mx = 0.0, pm = 0.0;  // quick_check starts from 1 and 0
     for (int b = 0; b < grid; ++b) {
