@@ -717,7 +717,6 @@ struct Mlp {
     uint16_t *wb = nullptr, *xf = nullptr, *gf = nullptr;
     float *sq = nullptr, *lparts = nullptr;
     long long frag_rows = 0, lparts_steps = 0;
-    char* pin = nullptr;                // pinned host staging of small queries (kPinBytes)
     long long step = 0;                 // AdamW step count
 };
 
@@ -725,13 +724,9 @@ constexpr int kPartBlocks = 256;
 // Query rows that go to the one-launch kernel: at most one 32-row block per CU;
 // with more rows its blocks re-read the weights where the 128-row blocks of the
 // inference kernel do so a quarter as often.  Two members of 256 x 4, host
-// arrays: 8 rows 75 -> 40 us, 2000 rows 118 -> 67, 8000 rows 216 -> 202; device
-// arrays: 8192 rows 47 -> 36.
+// arrays: 8 rows 70 -> 35 us, 2000 rows 108 -> 59, 8192 rows 195 -> 130; device
+// arrays: 8192 rows 43 -> 32.
 constexpr int64_t kQueryRowsMax = 8192;
-// Rows and results of up to this size together go through pinned host memory,
-// which the kernel reads and writes itself: without it 940 rows take 89 us
-// instead of 55, 8000 rows 207 instead of 202.
-constexpr size_t kPinBytes = 5 << 19;
 constexpr int kMaxSplits = 32;
 
 void dfree(void* q) {
@@ -748,7 +743,6 @@ void destroy(Mlp* n) {
     dfree(n->loss_hist); dfree(n->xin); dfree(n->xd); dfree(n->td); dfree(n->bidx);
     dfree(n->wpart); dfree(n->ens_spec); dfree(n->ens_spread); dfree(n->ts); dfree(n->wf);
     dfree(n->ey); dfree(n->wb); dfree(n->xf); dfree(n->gf); dfree(n->sq); dfree(n->lparts);
-    if (n->pin) (void)hipHostFree(n->pin);
     for (auto& e : n->ev)
         if (e) (void)hipEventDestroy(e);
     for (auto& e : n->tev)
@@ -1113,29 +1107,39 @@ bool device_memory(const void* q) {
 int query(Mlp* const* ms, int members, const float* x, int rows, double floor, float* spec,
           float* spread, bool dev) {
     Mlp* h = ms[0];
-    const size_t nx = 4 * (size_t)rows * h->cfg.nin, ny = 4 * (size_t)rows * h->cfg.nout, nr = 4 * (size_t)rows;
-    const bool pinned = !dev && nx + ny + nr <= kPinBytes;
+    const int nin = h->cfg.nin, nout = h->cfg.nout;
+    // Host rows and their results go through pinned slots, which the kernel reads
+    // and writes itself.  A slot takes at least 448 rows (16 inputs, 128 outputs).
+    // Against copies from and to pageable memory: 940 rows 89 -> 55 us, 5000 rows
+    // of 128 outputs 213 -> 152, 8192 rows 305 -> 229.
+    const int per = (int)(sp::kSlotBytes / (4 * (size_t)(nin + nout + 1) * sp::mlp::kQueryRows));
+    const int srows = per * sp::mlp::kQueryRows, nslots = dev ? 0 : (rows + srows - 1) / srows;
+    static_assert(kQueryRowsMax <= 448 * sp::PinnedSlots::kMax, "slots of a call");
     sp::mlp::QueryArgs a{};
     a.f = fused_args(ms, members);
     a.f.rows = rows;
     a.members = members;
-    a.nout = h->cfg.nout;
+    a.nout = nout;
     a.floor = (float)floor;
     a.f.x = x;
     a.spec = spec;
     a.spread = spread;
-    if (pinned) {
-        if (!h->pin) MLP_HIP(hipHostMalloc(reinterpret_cast<void**>(&h->pin), kPinBytes, hipHostMallocDefault));
-        a.spec = reinterpret_cast<float*>(h->pin);           // 16-byte rows first
-        a.spread = reinterpret_cast<float*>(h->pin + ny);
-        float* px = reinterpret_cast<float*>(h->pin + ny + nr);
-        std::memcpy(px, x, nx);
-        a.f.x = px;
-    } else if (!dev) {
-        MLP_HIP(hipMemcpyAsync(h->xin, x, nx, hipMemcpyHostToDevice, h->st));
-        a.f.x = h->xin;
-        a.spec = h->ens_spec;
-        a.spread = h->ens_spread;
+    int device = 0;
+    if (!dev) MLP_HIP(hipGetDevice(&device));
+    sp::PinnedSlots pin(device, h->st);
+    if (!dev) MLP_HIP(pin.take(nslots));
+    // slot k: its rows, and the places of their spectra, spreads and inputs
+    auto rows_of = [&](int k) { return (size_t)std::min(srows, rows - k * srows); };
+    auto place = [&](int k) { return static_cast<float*>(pin.slots()[k]); };
+    for (int k = 0; k < nslots; ++k) {
+        a.slot[k] = static_cast<char*>(pin.slots()[k]);
+        std::memcpy(place(k) + (size_t)srows * (nout + 1), x + (size_t)k * srows * nin, 4 * rows_of(k) * nin);
+    }
+    if (nslots > 1) a.per = per;
+    if (nslots == 1) {
+        a.spec = place(0);
+        a.spread = place(0) + (size_t)srows * nout;
+        a.f.x = a.spread + srows;
     }
     MLP_HIP(hipEventRecord(h->tev[0], h->st));
     const dim3 grid((unsigned)((rows + sp::mlp::kQueryRows - 1) / sp::mlp::kQueryRows));
@@ -1144,14 +1148,11 @@ int query(Mlp* const* ms, int members, const float* x, int rows, double floor, f
     else hipLaunchKernelGGL(sp::mlp::mlp_query_kernel<128>, grid, block, 0, h->st, a);
     MLP_HIP(hipGetLastError());
     MLP_HIP(hipEventRecord(h->tev[1], h->st));
-    if (!dev && !pinned) {
-        MLP_HIP(hipMemcpyAsync(spec, h->ens_spec, ny, hipMemcpyDeviceToHost, h->st));
-        MLP_HIP(hipMemcpyAsync(spread, h->ens_spread, nr, hipMemcpyDeviceToHost, h->st));
-    }
     MLP_HIP(hipStreamSynchronize(h->st));
-    if (pinned) {
-        std::memcpy(spec, a.spec, ny);
-        std::memcpy(spread, a.spread, nr);
+    pin.idle(true);
+    for (int k = 0; k < nslots; ++k) {
+        std::memcpy(spec + (size_t)k * srows * nout, place(k), 4 * rows_of(k) * nout);
+        std::memcpy(spread + (size_t)k * srows, place(k) + (size_t)srows * nout, 4 * rows_of(k));
     }
     float t = 0.f;
     MLP_HIP(hipEventElapsedTime(&t, h->tev[0], h->tev[1]));
@@ -1184,7 +1185,7 @@ int ensemble(void* const* nets, int32_t members, const float* x, int64_t rows, d
     const int nin = h->cfg.nin, nout = h->cfg.nout;
     const bool small = fused && rows > 0 && rows <= kQueryRowsMax && (dev || rows <= chunk) &&
                        2 * h->cfg.nhidden * members <= sp::mlp::kQueryThreads;
-    if (!dev && !h->ens_spec) {
+    if (!dev && !small && !h->ens_spec) {
         MLP_HIP(hipMalloc(&h->ens_spec, 4 * (size_t)h->bmax * nout));
         MLP_HIP(hipMalloc(&h->ens_spread, 4 * (size_t)h->bmax));
     }

@@ -7,8 +7,8 @@
 // as in train_rows_kernel: 32 features each, the next layer's weight fragments
 // in flight through the epilogue), and turns their outputs, left in LDS, into
 // mean spectrum and spread.  Inputs and results may lie in pinned host memory:
-// the rows are read once and each result is written once.  Every accumulation
-// and rounding is that of mlp_infer_kernel and ensemble_kernel.
+// each member's threads read the rows once and each result is written once.
+// Every accumulation and rounding is that of mlp_infer_kernel and ensemble_kernel.
 #pragma once
 
 namespace sp {
@@ -24,6 +24,10 @@ struct QueryArgs {
     float floor;
     float* spec;
     float* spread;
+    // per > 0: rows in several pinned slots (x, spec and spread then unused), of
+    // `per` blocks each: their spectra, spreads and inputs one after the other
+    int per;
+    char* slot[PinnedSlots::kMax];
 };
 
 template <int H>
@@ -36,8 +40,18 @@ __global__ void __launch_bounds__(kQueryThreads) mlp_query_kernel(QueryArgs a) {
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int g = wv / (H / 32), w = wv % (H / 32);       // member, wave of the member
     const int tid = threadIdx.x - g * 2 * H;
-    const long long r0 = (long long)blockIdx.x * kQueryRows;
-    const uint32_t mask = r0 + (lane & 31) < a.f.rows ? 0xFFFFFFFFu : 0u;
+    const int left = a.f.rows - (int)blockIdx.x * kQueryRows;   // rows from this block's first on
+    const float* x = a.f.x;
+    float *spec = a.spec, *spread = a.spread;
+    long long r0 = (long long)blockIdx.x * kQueryRows;          // first row in those arrays
+    if (a.per > 0) {
+        const int rows = a.per * kQueryRows;
+        spec = reinterpret_cast<float*>(a.slot[blockIdx.x / a.per]);
+        spread = spec + (long long)rows * a.nout;
+        x = spread + rows;
+        r0 = (long long)(blockIdx.x % a.per) * kQueryRows;
+    }
+    const uint32_t mask = (lane & 31) < left ? 0xFFFFFFFFu : 0u;
     const float* p = a.f.p[g];
     const v8bf* wf = reinterpret_cast<const v8bf*>(a.f.wf[g]);
     const int T = a.nout / 32, nl = a.f.nhh + 1;          // output tiles, hidden layers
@@ -51,7 +65,7 @@ __global__ void __launch_bounds__(kQueryThreads) mlp_query_kernel(QueryArgs a) {
     for (int i = 0; i < KSH; ++i) wq[i] = next[i * 64 + lane];
     for (int i = tid; i < kQueryRows * kFusedKin; i += 2 * H) {
         const int r = i / kFusedKin, c = i % kFusedKin;
-        const float v = (r0 + r < a.f.rows && c < a.f.nin) ? a.f.x[(r0 + r) * a.f.nin + c] : 0.0f;
+        const float v = (r < left && c < a.f.nin) ? x[(r0 + r) * a.f.nin + c] : 0.0f;
         act[g][0][r * LD + c] = bf16_rne(v);
     }
     v16f z;
@@ -90,7 +104,7 @@ __global__ void __launch_bounds__(kQueryThreads) mlp_query_kernel(QueryArgs a) {
     // ensemble_kernel on the outputs in LDS: 16 lanes per row
     const int l16 = threadIdx.x & 15;
     const float inv = 1.0f / (float)a.members;
-    for (int r = threadIdx.x >> 4; r < kQueryRows && r0 + r < a.f.rows; r += blockDim.x >> 4) {
+    for (int r = threadIdx.x >> 4; r < kQueryRows && r < left; r += blockDim.x >> 4) {
         float dist = 0.0f;
         for (int c = 4 * l16; c < a.nout; c += 64) {
             float4 yv[M];
@@ -113,11 +127,11 @@ __global__ void __launch_bounds__(kQueryThreads) mlp_query_kernel(QueryArgs a) {
                     if (i < a.members) dist += fabsf(sv[i] - mean);
                 mv[k] = mean;
             }
-            *reinterpret_cast<float4*>(a.spec + (r0 + r) * a.nout + c) = float4{mv[0], mv[1], mv[2], mv[3]};
+            *reinterpret_cast<float4*>(spec + (r0 + r) * a.nout + c) = float4{mv[0], mv[1], mv[2], mv[3]};
         }
 #pragma unroll
         for (int o = 8; o > 0; o >>= 1) dist += __shfl_xor(dist, o, 16);
-        if (l16 == 0) a.spread[r0 + r] = dist * inv;
+        if (l16 == 0) spread[r0 + r] = dist * inv;
     }
 }
 
