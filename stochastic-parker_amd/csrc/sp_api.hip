@@ -1565,24 +1565,25 @@ int sp_variant_distributions(void* ctx, int32_t nvar, double* fglobal, int64_t* 
     if (nvar < 1 || nvar > c->nvar) return fail(SP_ERR_ARG, "nvar must be in [1, number of installed variants]");
     const long long npp = c->da.npp;
     const size_t nbins = (size_t)npp * (size_t)nvar;
-    if (c->vhist_len < nbins + (size_t)nvar) {
+    // the counts begin on 16 bytes behind the bins, and reach the host with them
+    // (a copy of their own took 11 of 33 us)
+    const size_t cnt0 = nbins + (nbins & 1), len = cnt0 + (size_t)nvar;
+    if (c->vhist_len < len) {
         free_dev(c->vhist);
         c->vhist = nullptr;
         c->vhist_len = 0;
-        SP_HIP(hipMalloc(&c->vhist, sizeof(unsigned long long) * (nbins + (size_t)nvar)));
-        c->vhist_len = nbins + (size_t)nvar;
+        SP_HIP(hipMalloc(&c->vhist, sizeof(unsigned long long) * len));
+        c->vhist_len = len;
     }
     unsigned long long* hist = c->vhist;
-    unsigned long long* cnt = c->vhist + nbins;
-    SP_HIP(hipMemsetAsync(hist, 0, sizeof(unsigned long long) * (nbins + (size_t)nvar), c->st));
+    unsigned long long* cnt = c->vhist + cnt0;
+    SP_HIP(hipMemsetAsync(hist, 0, sizeof(unsigned long long) * len, c->st));
     SP_HIP(sp::launch_variant_dist(c->P[c->cur], c->nptl, c->da, nvar, hist, cnt, c->ncu, c->st));
-    std::vector<unsigned long long> hb(counts ? (size_t)nvar : 0);
-    if (counts)
-        SP_HIP(hipMemcpyAsync(hb.data(), cnt, sizeof(unsigned long long) * hb.size(), hipMemcpyDeviceToHost, c->st));
-    const BinsOut bins{hist, (long long)nbins, fglobal};
-    rc = read_bins(c, &bins, 1);   // ends with the stream idle
+    std::vector<double> hc(counts ? (size_t)nvar : 0);   // counts in units of kFxScale: exact
+    const BinsOut bins[2] = {{hist, (long long)nbins, fglobal}, {cnt, (long long)nvar, counts ? hc.data() : nullptr}};
+    rc = read_bins(c, bins, 2);
     if (rc != SP_OK) return rc;
-    for (size_t v = 0; v < hb.size(); ++v) counts[v] = (int64_t)hb[v];
+    for (size_t v = 0; v < hc.size(); ++v) counts[v] = (int64_t)(hc[v] * sp::kFxScale);
     return SP_OK;
 }
 
