@@ -713,7 +713,7 @@ struct Mlp {
     long long ey_rows = 0;
     std::vector<hipEvent_t> tev;        // per-chunk timing events of the fused launches
     // two-launch training steps: transposed weight fragments, the batch's
-    // activations and gradients, squared errors, loss partials per step
+    // activations and gradients, squared errors, loss partials of lparts_steps steps
     uint16_t *wb = nullptr, *xf = nullptr, *gf = nullptr;
     float *sq = nullptr, *lparts = nullptr;
     long long frag_rows = 0, lparts_steps = 0;
@@ -728,6 +728,8 @@ constexpr int kPartBlocks = 256;
 // arrays: 8192 rows 43 -> 32.
 constexpr int64_t kQueryRowsMax = 8192;
 constexpr int kMaxSplits = 32;
+// Steps of a training loop whose loss partials (1 KiB each) wait for their sum.
+constexpr int64_t kLossSteps = 4096;
 
 void dfree(void* q) {
     if (q) (void)hipFree(q);
@@ -1019,13 +1021,14 @@ int train_fused(Mlp* n, int64_t nsteps, int batch, double lr0, double lr_min, ui
         MLP_HIP(hipMalloc(&n->sq, 4 * (size_t)rows * c.nout));
         n->frag_rows = rows;
     }
-    if (n->lparts_steps < nsteps) {
+    const int64_t lsteps = std::min(nsteps, kLossSteps);
+    if (n->lparts_steps < lsteps) {
         dfree(n->lparts);
         n->lparts = nullptr;
         n->lparts_steps = 0;
         // and the step's AdamW scalars behind the last partials
-        MLP_HIP(hipMalloc(&n->lparts, 4 * ((size_t)nsteps * sp::mlp::kLossParts + 4)));
-        n->lparts_steps = nsteps;
+        MLP_HIP(hipMalloc(&n->lparts, 4 * ((size_t)lsteps * sp::mlp::kLossParts + 4)));
+        n->lparts_steps = lsteps;
     }
     int rc = refresh_frag(n, n->st);
     if (rc != SP_OK) return rc;
@@ -1067,16 +1070,16 @@ int train_fused(Mlp* n, int64_t nsteps, int batch, double lr0, double lr_min, ui
     for (int64_t s = 0; s < nsteps; ++s) {
         ra.step = (uint32_t)s;
         ra.t = (uint32_t)(n->step + s);
-        ua.loss_parts = n->lparts + s * sp::mlp::kLossParts;
+        ua.loss_parts = n->lparts + s % lsteps * sp::mlp::kLossParts;
         if (H == 256) launch_train_rows<256>(ra, nl, (unsigned)(rows / 32), n->st);
         else launch_train_rows<128>(ra, nl, (unsigned)(rows / 32), n->st);
         hipLaunchKernelGGL(sp::mlp::train_update_kernel, dim3(grid), dim3(sp::mlp::kUpdateBlock), 0, n->st, ua);
+        const int64_t q = s % lsteps + 1;   // steps whose partials wait
+        if (q == lsteps || s + 1 == nsteps)
+            hipLaunchKernelGGL(sp::mlp::train_loss_kernel, dim3((unsigned)q), dim3(256), 0, n->st, n->lparts,
+                               ra.scale, n->loss_hist + (s + 1 - q));
         MLP_HIP(hipGetLastError());
     }
-    if (nsteps > 0)
-        hipLaunchKernelGGL(sp::mlp::train_loss_kernel, dim3((unsigned)nsteps), dim3(256), 0, n->st, n->lparts,
-                           ra.scale, n->loss_hist);
-    MLP_HIP(hipGetLastError());
     return SP_OK;
 }
 
