@@ -401,18 +401,27 @@ int read_bins(Ctx* c, const BinsOut* arrays, int count) {
     return SP_OK;
 }
 
-// Key, index and digit-table scratch of the sorts, kept once allocated.
+// Key, index and digit-table scratch of the sorts, kept once allocated: all of
+// it or none.
 int sort_buffers(Ctx* c) {
-    const long long cap = particle_cap(c->nmax);
-    if (!c->skey[0]) {
-        const long long nt = std::max<long long>(1, sp::num_tiles(c->nmax));
-        for (int i = 0; i < 2; ++i) {
-            SP_HIP(hipMalloc(&c->skey[i], sizeof(uint32_t) * cap));
-            SP_HIP(hipMalloc(&c->sidx[i], sizeof(uint32_t) * cap));
-        }
-        SP_HIP(hipMalloc(&c->shist, sizeof(unsigned) * (1 << sp::kSortDigitBits) * (nt + 1)));
+    if (c->shist) return SP_OK;
+    const size_t bytes = sizeof(uint32_t) * (size_t)particle_cap(c->nmax);
+    const long long nt = std::max<long long>(1, sp::num_tiles(c->nmax));
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < 2 && e == hipSuccess; ++i) {
+        e = hipMalloc(&c->skey[i], bytes);
+        if (e == hipSuccess) e = hipMalloc(&c->sidx[i], bytes);
     }
-    return SP_OK;
+    if (e == hipSuccess) e = hipMalloc(&c->shist, sizeof(unsigned) * (1 << sp::kSortDigitBits) * (nt + 1));
+    if (e == hipSuccess) return SP_OK;
+    (void)hipGetLastError();   // the next launch would report it
+    for (int i = 0; i < 2; ++i) {
+        free_dev(c->skey[i]);
+        free_dev(c->sidx[i]);
+        c->skey[i] = c->sidx[i] = nullptr;
+    }
+    c->shist = nullptr;
+    return fail(SP_ERR_HIP, std::string("no memory for the sort's scratch: ") + hipGetErrorString(e));
 }
 
 // Orders the current particle set by the Morton key of 2^shift-cell blocks
@@ -1013,12 +1022,12 @@ int mover_run(Ctx* c, double t0, double dtf, int num_fine_steps, int nsteps_inte
         // fewer records, and the tail is short.
         const long long lanes = 256ll * ppl * grid;
         const bool wait = c->cfg.precision == SP_PREC_F32 && nrun > 5 * lanes;
-        const bool ordered = c->nvar > 1 && c->cfg.ndim == 2 && !ti && (fx & ~sp::FX_LEAN) == 0 && ppl == 1 &&
+        bool ordered = c->nvar > 1 && c->cfg.ndim == 2 && !ti && (fx & ~sp::FX_LEAN) == 0 && ppl == 1 &&
                              m.step_budget == 0u && nrun > lanes && (wait || nrun <= 16 * lanes);
+        // without memory for the order the particles run by index
+        ordered = ordered && sort_buffers(c) == SP_OK;
         if (ordered && wait) m.flags |= sp::MF_WAIT;
         if (ordered) {
-            rc = sort_buffers(c);
-            if (rc != SP_OK) return rc;
             uint32_t* digit = c->skey[0];
             if (c->cfg.precision == SP_PREC_F32H) SP_HIP(sp::launch_order_digit_f32h(m, ti, fx, c->cfg.ndim, digit, c->st));
             else if (c->cfg.precision == SP_PREC_F32) SP_HIP(sp::launch_order_digit_f32(m, ti, fx, c->cfg.ndim, digit, c->st));
