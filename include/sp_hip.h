@@ -119,7 +119,8 @@ typedef struct sp_mover_stats {
     int64_t nptl_escaped;   /* cumulative count of escaped particles */
     double leak;            /* cumulative weight leaked through open boundaries */
     double leak_negp;       /* cumulative weight removed for p < 0 */
-    double kernel_ms;       /* device time of the push kernel (HIP events, context stream) */
+    double kernel_ms;       /* device time of the push kernel and, in batches, of ordering its
+                               work (HIP events, context stream) */
     double total_ms;        /* device time of the whole call (push + boundary pass + removal) */
 } sp_mover_stats;
 

@@ -1006,6 +1006,9 @@ int mover_run(Ctx* c, double t0, double dtf, int num_fine_steps, int nsteps_inte
         m.part_len = (nrun + sp::kParts - 1) / sp::kParts;
         m.step_budget = nrun * 8 < c->nptl ? 0u : budget;
         const int grid = mover_grid(c, nrun, bpc, ppl);
+        // clear the work, step and pause counters (leak counters are cumulative)
+        SP_HIP(hipMemsetAsync(c->ctr, 0, offsetof(sp::Counters, leak_fx), c->st));
+        SP_HIP(hipEventRecord(c->ev[1], c->st));
         // Work order.  A batch mixes particles whose step counts differ by orders
         // of magnitude (kappa, and where kperp is small the drift, set the step);
         // handed out in spatial order, a long one that starts last runs on alone.
@@ -1035,9 +1038,6 @@ int mover_run(Ctx* c, double t0, double dtf, int num_fine_steps, int nsteps_inte
             SP_HIP(sp::launch_digit_order(digit, nrun, c->sidx[0], c->shist, c->st));
             m.order = c->sidx[0];
         }
-        // clear the work, step and pause counters (leak counters are cumulative)
-        SP_HIP(hipMemsetAsync(c->ctr, 0, offsetof(sp::Counters, leak_fx), c->st));
-        SP_HIP(hipEventRecord(c->ev[1], c->st));
         if (c->cfg.precision == SP_PREC_F32H) SP_HIP(sp::launch_mover_f32h(m, ti, fx, c->cfg.ndim, ppl, grid, c->st));
         else if (c->cfg.precision == SP_PREC_F32) SP_HIP(sp::launch_mover_f32(m, ti, fx, c->cfg.ndim, ppl, grid, c->st));
         else SP_HIP(sp::launch_mover_f64(m, ti, fx, c->cfg.ndim, grid, c->st));
