@@ -329,11 +329,12 @@ int mover_grid(Ctx* c, long long n, int bpc = 0, int ppl = 1) {
 }
 
 // Pinned results of one call, in one slot: quick_check partials, counters,
-// removal totals.
+// removal totals, predicted step counts.
 struct PinResults {
     double stats[5 * 1024];      // stats_grid rows
     sp::Counters ctr;
     unsigned long long totals[2];
+    float counts[sp::kOrderSample];
 };
 static_assert(sizeof(PinResults) <= sp::kSlotBytes, "fits a slot");
 
@@ -970,32 +971,94 @@ int sp_inject_particles_threshold(void* ctx, int32_t quantity, int64_t nptl, dou
     return SP_OK;
 }
 
+// Whether a batch of n particles on so many lanes gains by a work order, from a
+// sample of its predicted step counts.  A batch mixes particles whose step
+// counts differ by orders of magnitude (kappa, and where kperp is small the
+// drift, set the step); handed out in spatial order, a long one that starts last
+// runs on alone.  So the parts hand out those with the smaller first step
+// first: 64 variants, 1.2e6 particles on 512^2, 6.9 -> 5.0 ms (two intervals'
+// mean, FP32; FP64 14.2 -> 10.7).  Where all counts are alike that only costs
+// the order and its kernel's indirection (1.2e6 particles of 1000 steps 8.15 ->
+// 8.48 ms, 4e6 of 22 steps 1.54 -> 1.66).  So either
+//  - the longest chain is 3 times the mean: at 5 and more times the order gains
+//    12 to 30 % (6 to 20 particles a lane), at up to 2 times -2 to +1 %;
+//  - or 1.5 times, and half of a lane's load: FP64 2.3 a lane 4 %;
+//  - or, where the kernel's lanes wait for the wave's other work (MF_WAIT), the
+//    counts scatter: their mean deviation over the mean, times the particles
+//    a lane takes, is 0.8.  At 6 a lane 0.16 and 0.22 (0.98, 1.3) gain 5 %, 0.12 and
+//    0.10 (0.73, 0.6) lose 1 and 3 %; at 20 a lane 0.08 (1.7) gains 8 %.
+// The sample runs ahead of the spatial sort, and the host reads it meanwhile
+// (after the sort it took 20 us of an interval).
+// Lanes wait from 5 particles per lane up in FP32: 3.3 a lane 2 % slower
+// than the order alone, 4 2 %, 4.5 the same, 5 3 % faster, 6 5 %, 10 8 %.  Without
+// that the order gains up to 16 a lane (9 %) and loses 3 % at 44: the classes'
+// sparser windows of the sorted particles share fewer records, and the tail
+// is short.  Not below one particle per lane (nothing waits for a lane), and
+// not for single-variant runs: their steps differ little at the start, and in
+// 3D turbulence the first step does not tell (5-10 % slower).
+bool order_pays(const float* counts, double lanes, double n, bool wait) {
+    double sum = 0.0, top = 0.0, dev = 0.0;
+    auto at = [&](int k) { return counts[k] > 0.0f ? (double)counts[k] : 0.0; };   // 0 for a NaN
+    for (int k = 0; k < sp::kOrderSample; ++k) {
+        sum += at(k);
+        top = std::max(top, at(k));
+    }
+    const double mean = sum / sp::kOrderSample;
+    for (int k = 0; k < sp::kOrderSample; ++k) dev += std::fabs(at(k) - mean);
+    if (wait && dev * n >= 0.8 * sum * lanes) return true;
+    return top >= 3.0 * mean || (top >= 1.5 * mean && top * lanes >= 0.5 * mean * n);
+}
+
+// Steps per particle and launch of a mover run (sort_steps >= 0: a trial's).
+// With sort_steps, the interval runs as launches of at most sort_steps
+// steps per particle; between launches the paused particles are sorted
+// to the front in spatial order and the next launch takes only them.
+// Precedence, last wins: the configuration's sort_steps, the autotuner's
+// choice, SP_SORT_STEPS, an explicit trial value.
+unsigned mover_budget(const Ctx* c, int sort_steps) {
+    unsigned budget = (unsigned)c->cfg.sort_steps;
+    if (c->tuned_sort_steps >= 0) budget = (unsigned)c->tuned_sort_steps;
+    if (const char* e = std::getenv("SP_SORT_STEPS")) budget = (unsigned)std::max(0, std::atoi(e));
+    if (sort_steps >= 0) budget = (unsigned)sort_steps;
+    return c->cfg.sort_every <= 0 ? 0u : budget;
+}
+
+// Where a launch of the mover over n particles may take a work order (lanes:
+// those of its grid); its kernels are built for one-frame 2D steps.
+bool may_order(const Ctx* c, long long n, long long lanes, int ppl, unsigned budget, bool& wait) {
+    wait = c->cfg.precision == SP_PREC_F32 && n > 5 * lanes;
+    return c->nvar > 1 && c->cfg.ndim == 2 && !c->cfg.time_interp && (step_features(c->cfg) & ~sp::FX_LEAN) == 0 &&
+           ppl == 1 && budget == 0u && n > lanes && n >= sp::kOrderSample && (wait || n <= 16 * lanes);
+}
+
+// With counts, the sample of predicted step counts, and slot_ev[0] behind it;
+// else the digits of the work order.
+hipError_t launch_order(Ctx* c, const sp::MoverParams& m, uint32_t* digit, float* counts) {
+    const int fx = step_features(c->cfg), nd = c->cfg.ndim;
+    hipError_t e;
+    if (c->cfg.precision == SP_PREC_F32H) e = sp::launch_order_f32h(m, false, fx, nd, digit, counts, c->st);
+    else if (c->cfg.precision == SP_PREC_F32) e = sp::launch_order_f32(m, false, fx, nd, digit, counts, c->st);
+    else e = sp::launch_order_f64(m, false, fx, nd, digit, counts, c->st);
+    return e == hipSuccess && counts ? hipEventRecord(c->slot_ev[0], c->st) : e;
+}
+
 // The push of one interval: launches of the persistent mover over the
 // current particles, with re-sorts between launches when a step budget is set.
 // bpc > 0 / sort_steps >= 0 override the launch settings (autotuner trials).
 // With `deferred`, the steps and the time of a last launch without a budget
 // are left to the caller, who reads them after its own next synchronisation.
-// Counters pass through pr.
+// Counters pass through pr; `sampled`: the first launch's sample is on its way there.
 int mover_run(Ctx* c, double t0, double dtf, int num_fine_steps, int nsteps_interval, int bpc,
               int sort_steps, int ppl_trial, unsigned long long& steps, float& ms_push,
-              PinResults* pr, bool* deferred = nullptr) {
+              PinResults* pr, bool sampled = false, bool* deferred = nullptr) {
     const int ppl = mover_ppl(c, ppl_trial);
     int rc = SP_OK;
     const bool ti = c->cfg.time_interp != 0;
     const int fx = step_features(c->cfg);
-    // With sort_steps, the interval runs as launches of at most sort_steps
-    // steps per particle; between launches the paused particles are sorted
-    // to the front in spatial order and the next launch takes only them.
     // Once fewer than 1/8 of the particles are still moving, the last launch
     // runs them to the end of the interval: re-sorting a sparse remainder
     // costs more than its locality gains.
-    // Budget precedence, last wins: the configuration's sort_steps, the
-    // autotuner's choice, SP_SORT_STEPS, an explicit trial value.
-    unsigned budget = (unsigned)c->cfg.sort_steps;
-    if (c->tuned_sort_steps >= 0) budget = (unsigned)c->tuned_sort_steps;
-    if (const char* e = std::getenv("SP_SORT_STEPS")) budget = (unsigned)std::max(0, std::atoi(e));
-    if (sort_steps >= 0) budget = (unsigned)sort_steps;
-    if (c->cfg.sort_every <= 0) budget = 0u;
+    const unsigned budget = mover_budget(c, sort_steps);
     steps = 0;
     ms_push = 0.f;
     long long nrun = c->nptl;
@@ -1009,32 +1072,19 @@ int mover_run(Ctx* c, double t0, double dtf, int num_fine_steps, int nsteps_inte
         // clear the work, step and pause counters (leak counters are cumulative)
         SP_HIP(hipMemsetAsync(c->ctr, 0, offsetof(sp::Counters, leak_fx), c->st));
         SP_HIP(hipEventRecord(c->ev[1], c->st));
-        // Work order.  A batch mixes particles whose step counts differ by orders
-        // of magnitude (kappa, and where kperp is small the drift, set the step);
-        // handed out in spatial order, a long one that starts last runs on alone.
-        // So the parts hand out those with the smaller first step first: 64
-        // variants, 1.2e6 particles on 512^2, 6.9 -> 5.0 ms (two intervals'
-        // mean, FP32; FP64 14.2 -> 10.7).  Not below one particle per lane
-        // (nothing waits for a lane), and not for single-variant runs: their
-        // steps differ little at the start, and in 3D turbulence the first step
-        // does not tell (5-10 % slower).  The FP32 kernel's lanes wait for the
-        // wave's other work (MF_WAIT) from 5 particles per lane up: 3.3 a lane
-        // 15 % slower, 6 a lane 8 % faster, 19 a lane 14 %, 80 a lane 62.5 ->
-        // 54.4 ms.  Without that the order gains up to 16 a lane (9 %) and loses
-        // 3 % at 44: the classes' sparser windows of the sorted particles share
-        // fewer records, and the tail is short.
+        // a batch's work order, where it pays and there is memory for it
         const long long lanes = 256ll * ppl * grid;
-        const bool wait = c->cfg.precision == SP_PREC_F32 && nrun > 5 * lanes;
-        bool ordered = c->nvar > 1 && c->cfg.ndim == 2 && !ti && (fx & ~sp::FX_LEAN) == 0 && ppl == 1 &&
-                             m.step_budget == 0u && nrun > lanes && (wait || nrun <= 16 * lanes);
-        // without memory for the order the particles run by index
-        ordered = ordered && sort_buffers(c) == SP_OK;
-        if (ordered && wait) m.flags |= sp::MF_WAIT;
+        bool wait, ordered = may_order(c, nrun, lanes, ppl, m.step_budget, wait);
         if (ordered) {
+            if (!sampled) SP_HIP(launch_order(c, m, nullptr, pr->counts));
+            SP_HIP(hipEventSynchronize(c->slot_ev[0]));
+            ordered = order_pays(pr->counts, (double)lanes, (double)nrun, wait) && sort_buffers(c) == SP_OK;
+        }
+        sampled = false;
+        if (ordered) {
+            if (wait) m.flags |= sp::MF_WAIT;
             uint32_t* digit = c->skey[0];
-            if (c->cfg.precision == SP_PREC_F32H) SP_HIP(sp::launch_order_digit_f32h(m, ti, fx, c->cfg.ndim, digit, c->st));
-            else if (c->cfg.precision == SP_PREC_F32) SP_HIP(sp::launch_order_digit_f32(m, ti, fx, c->cfg.ndim, digit, c->st));
-            else SP_HIP(sp::launch_order_digit_f64(m, ti, fx, c->cfg.ndim, digit, c->st));
+            SP_HIP(launch_order(c, m, digit, nullptr));
             SP_HIP(sp::launch_digit_order(digit, nrun, c->sidx[0], c->shist, c->st));
             m.order = c->sidx[0];
         }
@@ -1077,6 +1127,15 @@ int sp_particle_mover(void* ctx, double t0, double dtf, int32_t num_fine_steps,
     PinResults* const pr = static_cast<PinResults*>(pin.slots()[0]);
     const bool sorting = c->cfg.sort_every > 0;
     SP_HIP(hipEventRecord(c->ev[0], c->st));
+    const int ppl = mover_ppl(c);
+    bool wait;
+    const bool sampled = may_order(c, c->nptl, 256ll * ppl * mover_grid(c, c->nptl, 0, ppl), ppl,
+                                   mover_budget(c, -1), wait);
+    if (sampled) {
+        sp::MoverParams m = mover_params(c, t0, dtf, num_fine_steps, nsteps_interval);
+        m.n = c->nptl;
+        SP_HIP(launch_order(c, m, nullptr, pr->counts));
+    }
     if (sorting && c->mover_calls % c->cfg.sort_every == 0) {
         rc = spatial_sort(c);
         if (rc != SP_OK) return rc;
@@ -1085,7 +1144,7 @@ int sp_particle_mover(void* ctx, double t0, double dtf, int32_t num_fine_steps,
     unsigned long long steps = 0;
     float ms_push = 0.f;
     bool deferred = false;
-    rc = mover_run(c, t0, dtf, num_fine_steps, nsteps_interval, 0, -1, 0, steps, ms_push, pr, &deferred);
+    rc = mover_run(c, t0, dtf, num_fine_steps, nsteps_interval, 0, -1, 0, steps, ms_push, pr, sampled, &deferred);
     if (rc != SP_OK) return rc;
     // remove_particles: stable compaction into the other buffer set
     long long kept = 0, esc = 0;

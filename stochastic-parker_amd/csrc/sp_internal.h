@@ -321,9 +321,15 @@ hipError_t launch_step_once_f64(const MoverParams& m, bool ti, int fx, int ndim,
 hipError_t launch_step_once_f32(const MoverParams& m, bool ti, int fx, int ndim, const StepRows& r,
                                 hipStream_t s);
 
-// digit[i]: mover part and predicted step-count class of particle i
-hipError_t launch_order_digit_f64(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit, hipStream_t s);
-hipError_t launch_order_digit_f32(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit, hipStream_t s);
-hipError_t launch_order_digit_f32h(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit, hipStream_t s);
+// With counts: the predicted step counts of kOrderSample particles (m.n is at
+// least that).  Without: digit[i] = mover part and predicted step-count class
+// of particle i.
+constexpr int kOrderSample = 2048;
+hipError_t launch_order_f64(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit, float* counts,
+                            hipStream_t s);
+hipError_t launch_order_f32(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit, float* counts,
+                            hipStream_t s);
+hipError_t launch_order_f32h(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit, float* counts,
+                             hipStream_t s);
 
 }  // namespace sp

@@ -97,12 +97,14 @@ hipError_t launch_step_once_f32(const MoverParams& m, bool ti, int fx, int ndim,
     return launch_step_once<PolicyF32>(m, ti, fx, ndim, r, s);
 }
 
-hipError_t launch_order_digit_f32(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit, hipStream_t s) {
-    return launch_order_digit<PolicyF32>(m, ti, fx, ndim, digit, s);
+hipError_t launch_order_f32(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit, float* counts,
+                            hipStream_t s) {
+    return launch_order<PolicyF32>(m, ti, fx, ndim, digit, counts, s);
 }
 
-hipError_t launch_order_digit_f32h(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit, hipStream_t s) {
-    return launch_order_digit<PolicyF32H>(m, ti, fx, ndim, digit, s);
+hipError_t launch_order_f32h(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit, float* counts,
+                            hipStream_t s) {
+    return launch_order<PolicyF32H>(m, ti, fx, ndim, digit, counts, s);
 }
 
 }  // namespace sp

@@ -55,8 +55,9 @@ hipError_t launch_step_once_f64(const MoverParams& m, bool ti, int fx, int ndim,
     return launch_step_once<PolicyF64>(m, ti, fx, ndim, r, s);
 }
 
-hipError_t launch_order_digit_f64(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit, hipStream_t s) {
-    return launch_order_digit<PolicyF64>(m, ti, fx, ndim, digit, s);
+hipError_t launch_order_f64(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit, float* counts,
+                            hipStream_t s) {
+    return launch_order<PolicyF64>(m, ti, fx, ndim, digit, counts, s);
 }
 
 }  // namespace sp

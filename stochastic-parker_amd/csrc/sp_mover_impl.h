@@ -490,14 +490,9 @@ __global__ void __launch_bounds__(kStepRows) step_once_kernel(MoverParams m, Ste
     }
 }
 
-// Part of each particle (m.part_len) and the class of the step count that its
-// first step's dt predicts, the larger counts first: classes a factor of two
-// apart from the smallest count, dtf / dt_max, up.  digit = part * 8 + class.
-constexpr int kOrderClasses = 8;
+// dt that particle i's first step would take, by a step with zero increments.
 template <class Pol, int NDIM, bool TINTERP, int FX>
-__global__ void __launch_bounds__(256) order_digit_kernel(MoverParams m, uint32_t* digit) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m.n) return;
+__device__ __forceinline__ double first_dt(MoverParams& m, long long i) {
     State s{m.P.d(PD_X)[i], m.P.d(PD_Y)[i], m.P.d(PD_Z)[i], m.P.d(PD_P)[i], m.P.d(PD_T)[i], m.P.d(PD_DT)[i], 0.0};
     if constexpr ((FX & FX_NLGC) != 0) s.mu = m.P.d(PD_MU)[i];
     typename Pol::Var var = Pol::var_of(m);
@@ -508,9 +503,30 @@ __global__ void __launch_bounds__(256) order_digit_kernel(MoverParams m, uint32_
     const double still[4] = {0.0, 0.0, 0.0, 0.0};
     double d[4];
     Pol::template step_given<NDIM, TINTERP, FX>(m, var, s, false, still, d);
-    const float c = __builtin_amdgcn_logf((float)m.dt_max / (float)s.dt);   // log2; a NaN goes last
+    return s.dt;
+}
+
+// Part of each particle (m.part_len) and the class of the step count that its
+// first step's dt predicts, the larger counts first: classes a factor of two
+// apart from the smallest count, dtf / dt_max, up.  digit = part * 8 + class.
+constexpr int kOrderClasses = 8;
+template <class Pol, int NDIM, bool TINTERP, int FX>
+__global__ void __launch_bounds__(256) order_digit_kernel(MoverParams m, uint32_t* digit) {
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= m.n) return;
+    const double dt = first_dt<Pol, NDIM, TINTERP, FX>(m, i);
+    const float c = __builtin_amdgcn_logf((float)m.dt_max / (float)dt);   // log2; a NaN goes last
     const int few = c > 0.0f ? (int)fminf(c, (float)(kOrderClasses - 1)) : 0;
     digit[i] = (uint32_t)(i / m.part_len) * kOrderClasses + (uint32_t)(kOrderClasses - 1 - few);
+}
+
+// Predicted step counts of kOrderSample particles spread over the population
+// (at least as many), into pinned memory.
+template <class Pol, int NDIM, bool TINTERP, int FX>
+__global__ void __launch_bounds__(256) order_sample_kernel(MoverParams m, float* counts) {
+    const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    const double dt = first_dt<Pol, NDIM, TINTERP, FX>(m, t * (m.n / kOrderSample));
+    counts[t] = (float)(m.dtf / dt);
 }
 
 template <int N, bool T, int X>
@@ -619,15 +635,21 @@ hipError_t launch_mover(const MoverParams& m, bool ti, int fx, int ndim, int ppl
 }
 
 template <class Pol>
-hipError_t launch_order_digit(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit,
-                              hipStream_t st) {
-    if (m.n <= 0) return hipSuccess;
-    const int grid = (int)((m.n + 255) / 256);
+hipError_t launch_order(const MoverParams& m, bool ti, int fx, int ndim, uint32_t* digit, float* counts,
+                        hipStream_t st) {
+    static_assert(kOrderSample % 256 == 0, "whole blocks");
+    if (m.n < (counts ? kOrderSample : 1)) return hipErrorInvalidValue;
+    const int grid = counts ? kOrderSample / 256 : (int)((m.n + 255) / 256);
     const int built = dispatch_variant<Pol>(ndim, ti, fx, [&](auto v) {
         using V = decltype(v);
-        if constexpr (kOrdered<V>)
-            hipLaunchKernelGGL((order_digit_kernel<Pol, V::ndim, V::ti, V::fx>), dim3(grid), dim3(256), 0, st,
-                               m, digit);
+        if constexpr (kOrdered<V>) {
+            if (counts)
+                hipLaunchKernelGGL((order_sample_kernel<Pol, V::ndim, V::ti, V::fx>), dim3(grid), dim3(256), 0,
+                                   st, m, counts);
+            else
+                hipLaunchKernelGGL((order_digit_kernel<Pol, V::ndim, V::ti, V::fx>), dim3(grid), dim3(256), 0,
+                                   st, m, digit);
+        }
         return kOrdered<V> ? 1 : 0;
     });
     return built ? hipGetLastError() : hipErrorInvalidValue;
