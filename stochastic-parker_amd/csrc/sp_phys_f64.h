@@ -21,13 +21,24 @@ namespace f64 {
 // second then rounds correctly (P. Markstein, "Computation of elementary
 // functions on the IBM RISC System/6000 processor", 1990).  Five instructions
 // instead of twelve for the constant denominators dx, dy, dz, p0, dtf and 3
-// (an infinite a gives NaN; quotient and residuals must not underflow).  With
-// the merged quotients of the dt rule below: 2000 particles on 64^2 42.7 ->
-// 36.5 ms per interval at equal work.
-__device__ __forceinline__ double div_const(double a, double b, double rb) {
+// (quotient and residuals must not underflow).  With the merged quotients of
+// the dt rule below: 2000 particles on 64^2 42.7 -> 36.5 ms per interval at
+// equal work.  An infinite a gives NaN here: enough for a cell offset, which an
+// infinite position makes NaN anyway.
+__device__ __forceinline__ double div_finite(double a, double b, double rb) {
     double q = a * rb;
     q = fma(fma(-b, q, a), rb, q);
     return fma(fma(-b, q, a), rb, q);
+}
+// The same with IEEE results for infinite a, for overflow and for zeros' signs:
+// one instruction more.
+__device__ __forceinline__ double div_const(double a, double b, double rb) {
+    const double q = div_finite(a, b, rb);
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_div_fixup(q, b, a);
+#else
+    return q;
+#endif
 }
 
 // get_interp_paramters (particle_module.f90:642-674) on a uniform grid:
@@ -40,8 +51,8 @@ struct Interp {
 template <int NDIM>
 __device__ __forceinline__ Interp interp_params(const MoverParams& m, double x, double y, double z) {
     Interp I;
-    const double px = div_const(x - m.xmin, m.dx, m.idx);
-    const double py = div_const(y - m.ymin, m.dy, m.idy);
+    const double px = div_finite(x - m.xmin, m.dx, m.idx);
+    const double py = div_finite(y - m.ymin, m.dy, m.idy);
     const double fx = floor(px), fy = floor(py);
     const double rx = (px - (fx + 1.0)) + 1.0;  // px - pos + 1 with pos = floor(px) + 1
     const double ry = (py - (fy + 1.0)) + 1.0;
@@ -50,7 +61,7 @@ __device__ __forceinline__ Interp interp_params(const MoverParams& m, double x, 
     I.iy = step_cell(fy, m.nyg - 4) + 2;
     I.iz = 0;
     if (NDIM == 3) {
-        const double pz = div_const(z - m.zmin, m.dz, m.idz);
+        const double pz = div_finite(z - m.zmin, m.dz, m.idz);
         const double fz = floor(pz);
         rz = (pz - (fz + 1.0)) + 1.0;
         I.iz = step_cell(fz, m.nzg - 4) + 2;
