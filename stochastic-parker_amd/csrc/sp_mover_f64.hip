@@ -31,13 +31,13 @@ struct PolicyF64 {
                                                 double d[4], GC& gc) {
         double r[4];
         f64::step_rands(m, rng, rstep, r);
-        f64::gather_kappa_push<NDIM, TI, FX>(m, s, fixed, r, d, gc);
+        f64::gather_kappa_push<NDIM, TI, FX, false>(m, s, fixed, r, d, gc);
     }
     template <int NDIM, bool TI, int FX>
     __device__ __forceinline__ static void step_given(const MoverParams& m, const Var&, State& s,
                                                       bool fixed, const double* r, double d[4]) {
         f64::CellCache<false> none;
-        f64::gather_kappa_push<NDIM, TI, FX>(m, s, fixed, r, d, none);
+        f64::gather_kappa_push<NDIM, TI, FX, true>(m, s, fixed, r, d, none);
     }
 };
 

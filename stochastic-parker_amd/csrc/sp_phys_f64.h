@@ -434,8 +434,10 @@ __device__ __forceinline__ void dpp_terms(const MoverParams& m, double p, const 
 // (:4625-4907), Cartesian, uniform grid; the momentum-diffusion terms when FX
 // has FX_DPP.  r = (ran1, ran2, ran3, ran_p).  d receives (deltax, deltay,
 // deltaz, deltap); the 2D pusher leaves deltaz at zero like the reference (its
-// z drift is not undone).
-template <int NDIM, int FX>
+// z drift is not undone).  GIVEN: increments and time step are a caller's and
+// may be anything, so the momentum's noise term is formed where it is zero too
+// (an infinite increment or a negative time step makes it NaN).
+template <int NDIM, int FX, bool GIVEN>
 __device__ __forceinline__ void push(const MoverParams& m, State& s, const double* f,
                                      const Kappa& k, bool fixed_dt, const double r[4],
                                      double d[4]) {
@@ -534,6 +536,7 @@ __device__ __forceinline__ void push(const MoverParams& m, State& s, const doubl
     s.t = s.t + s.dt;
     double dp = dp_dt * s.dt;
     if constexpr ((FX & FX_DPP) != 0) dp = dp + r[3] * sqrt(2.0 * dpp) * sdt;
+    else if constexpr (GIVEN) dp = dp + r[3] * 0.0 * sdt;
     if (ACC) {
         if (in_acc_region<NDIM>(m, s.x, s.y, s.z)) s.p = s.p + dp;
         else dp = 0.0;
@@ -564,7 +567,7 @@ __device__ __forceinline__ void step_rands(const MoverParams& m, const PhiloxPtl
 }
 
 // The full per-step chain: interpolation parameters, gather, kappa, push.
-template <int NDIM, bool TINTERP, int FX, class GC>
+template <int NDIM, bool TINTERP, int FX, bool GIVEN, class GC>
 __device__ __forceinline__ void gather_kappa_push(const MoverParams& m, State& s, bool fixed_dt,
                                                   const double r[4], double d[4], GC& gc) {
     constexpr bool DPP = (FX & FX_DPP) != 0;
@@ -575,7 +578,7 @@ __device__ __forceinline__ void gather_kappa_push(const MoverParams& m, State& s
     Kappa k;
     if constexpr ((FX & FX_NLGC) != 0) k = kappa_nlgc<NDIM>(m, s.p, s.mu, f);
     else k = kappa<NDIM>(m, s.p, f);
-    push<NDIM, FX>(m, s, f, k, fixed_dt, r, d);
+    push<NDIM, FX, GIVEN>(m, s, f, k, fixed_dt, r, d);
 }
 
 }  // namespace f64

@@ -1,6 +1,7 @@
 """FP64 steps with operands that are not finite or too large, against the
 oracle bit for bit (signs of zeros aside): infinite and huge momenta,
-infinite times, gradients that overflow."""
+infinite times, gradients that overflow; increments and given time steps that
+are infinite, NaN or negative."""
 import numpy as np
 import pytest
 
@@ -59,3 +60,23 @@ def test_infinite_momentum_with_kappas_momentum_dependence(ndim):
     a["p"] = np.inf
     r = np.random.default_rng(1).uniform(-1.7, 1.7, (len(a), 4))
     compare(c, [nodes_for(c)], a, r, np.zeros(len(a), np.int8))
+
+
+@pytest.mark.parametrize("acc", [0, 1])
+@pytest.mark.parametrize("ndim,n", [(2, 33), (3, 11)])
+def test_steps_with_special_increments(ndim, n, acc):
+    c = (cfg2d if ndim == 2 else cfg3d)(n, momentum_dependency=0, mag_dependency=0, p0=1.3, acc_region_flag=acc,
+                                        acc_region=(0.0, 0.5, 0.0, 1.0, 0.0, 1.0))
+    a = random_states(c, 800, seed=8)
+    rng = np.random.default_rng(ndim)
+    k = np.arange(len(a)) % 8
+    r = rng.uniform(-1.7, 1.7, (len(a), 4))
+    r[k == 1, 3] = np.inf
+    r[k == 2, 3] = np.nan
+    r[k == 3, 0] = np.inf
+    fixed = (rng.random(len(a)) < 0.2).astype(np.int8)
+    fixed[k >= 4] = 1
+    a["dt"][k == 4] = -1e-5
+    a["dt"][k == 5] = np.inf
+    a["dt"][k == 6] = np.nan
+    compare(c, [nodes_for(c)], a, r, fixed)
