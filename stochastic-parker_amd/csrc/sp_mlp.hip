@@ -1004,32 +1004,50 @@ void launch_train_rows(const sp::mlp::RowsArgs& a, int nl, unsigned grid, hipStr
     else go(sp::mlp::train_rows_kernel<H, 5>);
 }
 
+// Its memory for batches of `batch` rows, kept for later calls.  False where
+// there is none: the layer kernels, which need only what the network has, serve
+// instead.
+bool train_buffers(Mlp* n, int64_t nsteps, int batch) {
+    const sp_mlp_config& c = n->cfg;
+    const long long rows = (batch + 31) / 32 * 32;
+    const sp::mlp::RowFrags fr{(int)(rows / 16), c.nhidden / 32};
+    hipError_t e = hipSuccess;
+    if (!n->wb) e = hipMalloc(&n->wb, 2 * (size_t)c.nlayers * c.nhidden * c.nhidden);
+    if (e == hipSuccess && n->frag_rows < rows) {
+        dfree(n->xf); dfree(n->gf); dfree(n->sq);
+        n->xf = n->gf = nullptr;
+        n->sq = nullptr;
+        n->frag_rows = 0;
+        e = hipMalloc(&n->xf, 2 * (size_t)fr.x(n->L));
+        if (e == hipSuccess) e = hipMalloc(&n->gf, 2 * (size_t)(fr.g(c.nlayers) + 16ll * fr.rs * c.nout));
+        if (e == hipSuccess) e = hipMalloc(&n->sq, 4 * (size_t)rows * c.nout);
+        if (e == hipSuccess) n->frag_rows = rows;
+    }
+    const long long lsteps = std::min(nsteps, kLossSteps);
+    if (e == hipSuccess && n->lparts_steps < lsteps) {
+        dfree(n->lparts);
+        n->lparts = nullptr;
+        n->lparts_steps = 0;
+        // and the step's AdamW scalars behind the last partials
+        e = hipMalloc(&n->lparts, 4 * ((size_t)lsteps * sp::mlp::kLossParts + 4));
+        if (e == hipSuccess) n->lparts_steps = lsteps;
+    }
+    if (e == hipSuccess) return true;
+    (void)hipGetLastError();   // the next launch would report it
+    if (n->frag_rows == 0) {
+        dfree(n->xf); dfree(n->gf);
+        n->xf = n->gf = nullptr;
+    }
+    return false;
+}
+
 int train_fused(Mlp* n, int64_t nsteps, int batch, double lr0, double lr_min, uint64_t seed) {
     static_assert(sp::mlp::kUpdateSplits == kMaxSplits && sp::mlp::kLossParts == kPartBlocks, "layer path's orders");
     const sp_mlp_config& c = n->cfg;
     const int H = c.nhidden, nl = c.nlayers, L = n->L;
     const long long rows = (batch + 31) / 32 * 32;
     const sp::mlp::RowFrags fr{(int)(rows / 16), H / 32};
-    if (!n->wb) MLP_HIP(hipMalloc(&n->wb, 2 * (size_t)nl * H * H));
-    if (n->frag_rows < rows) {
-        dfree(n->xf); dfree(n->gf); dfree(n->sq);
-        n->xf = n->gf = nullptr;
-        n->sq = nullptr;
-        n->frag_rows = 0;
-        MLP_HIP(hipMalloc(&n->xf, 2 * (size_t)fr.x(L)));
-        MLP_HIP(hipMalloc(&n->gf, 2 * (size_t)(fr.g(nl) + 16ll * fr.rs * c.nout)));
-        MLP_HIP(hipMalloc(&n->sq, 4 * (size_t)rows * c.nout));
-        n->frag_rows = rows;
-    }
     const int64_t lsteps = std::min(nsteps, kLossSteps);
-    if (n->lparts_steps < lsteps) {
-        dfree(n->lparts);
-        n->lparts = nullptr;
-        n->lparts_steps = 0;
-        // and the step's AdamW scalars behind the last partials
-        MLP_HIP(hipMalloc(&n->lparts, 4 * ((size_t)lsteps * sp::mlp::kLossParts + 4)));
-        n->lparts_steps = lsteps;
-    }
     int rc = refresh_frag(n, n->st);
     if (rc != SP_OK) return rc;
     for (int l = 1; l < L; ++l) {
@@ -1529,7 +1547,7 @@ int sp_mlp_train(void* q, int64_t nsteps, int32_t batch, double lr0, double lr_m
     };
     const char* eager_env = std::getenv("SP_MLP_EAGER");
     const bool eager = eager_env && std::atoi(eager_env) != 0;
-    if (!eager && train_fused_ok(n)) {
+    if (!eager && train_fused_ok(n) && train_buffers(n, nsteps, batch)) {
         rc = train_fused(n, nsteps, batch, lr0, lr_min, seed);
         if (rc != SP_OK) return rc;
         n->fver = n->pver;   // the update kernel keeps wf with the weights
