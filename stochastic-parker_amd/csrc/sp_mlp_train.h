@@ -417,7 +417,8 @@ __global__ void __launch_bounds__(kUpdateBlock) train_update_kernel(UpdateArgs a
         if (b >= N / 32) { b -= N / 32; continue; }
         const uint16_t* G = a.gf + a.fr.g(l) + (long long)b * rs * 512;
         const int chunk = (a.rows + kColParts - 1) / kColParts;
-        static_assert(kColParts * 32 <= kUpdateSplits * 32, "partial sums fit in LDS");
+        static_assert(2 * kColParts <= kUpdateSplits, "each row chunk's 32 x 32 phase sums take two rows of part");
+        static_assert(kColParts * 32 <= kUpdateBlock, "one thread per chunk and column");
         if (chunk % 32 == 0) {
             // whole 32-row groups (zeros past the batch): eight phases per load
             for (int i = t; i < kColParts * 128; i += kUpdateBlock) {
