@@ -231,7 +231,9 @@ int sp_split_particle(void* ctx, double split_ratio, double pmin_split);
  * (x, y, z, p, t, dt) per particle and are updated in place; deltas receives
  * (dx, dy, dz, dp) per particle.  fixed_dt is per particle (0/1).  With nlgc,
  * row i takes its pitch-angle cosine mu from the context's particle i
- * (n <= nptl_current). */
+ * (n <= nptl_current).  Rows go through pinned staging in pieces: without
+ * memory for it the call fails before any row is touched; a device error
+ * may leave the first rows stepped and the others as they were. */
 int sp_step_once(void* ctx, int64_t n, double t0, double dtf, double* state,
                  const double* rands, const int8_t* fixed_dt, double* deltas);
 /* No counterpart in the reference.  sp_step_once without device allocation,

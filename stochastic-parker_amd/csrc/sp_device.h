@@ -68,7 +68,7 @@ __device__ __forceinline__ U4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c
 }
 
 // The steps of one particle differ in counter word 2 (the step) alone, so
-// three of the first two rounds' four products and their XORs belong to the
+// two of the first two rounds' four products and their XORs belong to the
 // particle: formed once when a lane takes it (18 products a step instead of
 // 20).  With step_cell, the momentum floor's branch and ballots without their
 // integer detour, 25 of 310 vector instructions of a 2D FP32 step: 2e7
