@@ -28,6 +28,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "sp_device.h"
@@ -1136,11 +1137,12 @@ int query(Mlp* const* ms, int members, const float* x, int rows, double floor, f
     const int per = (int)(sp::kSlotBytes / (4 * (size_t)(nin + nout + 1) * sp::mlp::kQueryRows));
     const int srows = per * sp::mlp::kQueryRows, nslots = dev ? 0 : (rows + srows - 1) / srows;
     static_assert(kQueryRowsMax <= 448 * sp::PinnedSlots::kMax, "slots of a call");
-    sp::mlp::QueryArgs a{};
+    sp::mlp::QueryPieces a{};
     a.f = fused_args(ms, members);
     a.f.rows = rows;
     a.members = members;
     a.nout = nout;
+    a.per = per;
     a.floor = (float)floor;
     a.f.x = x;
     a.spec = spec;
@@ -1156,7 +1158,6 @@ int query(Mlp* const* ms, int members, const float* x, int rows, double floor, f
         a.slot[k] = static_cast<char*>(pin.slots()[k]);
         std::memcpy(place(k) + (size_t)srows * (nout + 1), x + (size_t)k * srows * nin, 4 * rows_of(k) * nin);
     }
-    if (nslots > 1) a.per = per;
     if (nslots == 1) {
         a.spec = place(0);
         a.spread = place(0) + (size_t)srows * nout;
@@ -1165,8 +1166,13 @@ int query(Mlp* const* ms, int members, const float* x, int rows, double floor, f
     MLP_HIP(hipEventRecord(h->tev[0], h->st));
     const dim3 grid((unsigned)((rows + sp::mlp::kQueryRows - 1) / sp::mlp::kQueryRows));
     const dim3 block((unsigned)(2 * h->cfg.nhidden * members));
-    if (h->cfg.nhidden == 256) hipLaunchKernelGGL(sp::mlp::mlp_query_kernel<256>, grid, block, 0, h->st, a);
-    else hipLaunchKernelGGL(sp::mlp::mlp_query_kernel<128>, grid, block, 0, h->st, a);
+    auto go = [&](const auto& args) {
+        using Args = std::decay_t<decltype(args)>;
+        if (h->cfg.nhidden == 256) hipLaunchKernelGGL((sp::mlp::mlp_query_kernel<256, Args>), grid, block, 0, h->st, args);
+        else hipLaunchKernelGGL((sp::mlp::mlp_query_kernel<128, Args>), grid, block, 0, h->st, args);
+    };
+    if (nslots > 1) go(a);
+    else go(static_cast<const sp::mlp::QueryArgs&>(a));
     MLP_HIP(hipGetLastError());
     MLP_HIP(hipEventRecord(h->tev[1], h->st));
     MLP_HIP(hipStreamSynchronize(h->st));

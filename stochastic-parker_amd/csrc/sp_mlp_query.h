@@ -24,14 +24,18 @@ struct QueryArgs {
     float floor;
     float* spec;
     float* spread;
-    // per > 0: rows in several pinned slots (x, spec and spread then unused), of
-    // `per` blocks each: their spectra, spreads and inputs one after the other
+};
+
+// Rows in several pinned slots (x, spec and spread then unused), of `per` blocks
+// each: their spectra, spreads and inputs one after the other.  Arguments of a
+// kernel of its own, which other queries do not wait for (0.5 us).
+struct QueryPieces : QueryArgs {
     int per;
     char* slot[PinnedSlots::kMax];
 };
 
-template <int H>
-__global__ void __launch_bounds__(kQueryThreads) mlp_query_kernel(QueryArgs a) {
+template <int H, class Args>
+__global__ void __launch_bounds__(kQueryThreads) mlp_query_kernel(Args a) {
     constexpr int M = kQueryThreads / (2 * H), LD = H + 8, KSH = H / 16, LY = 128 + 4;
     static_assert(M <= kQueryMembers, "members of a block");
     __shared__ __align__(16) uint16_t act[M][2][kQueryRows * LD];
@@ -44,7 +48,7 @@ __global__ void __launch_bounds__(kQueryThreads) mlp_query_kernel(QueryArgs a) {
     const float* x = a.f.x;
     float *spec = a.spec, *spread = a.spread;
     long long r0 = (long long)blockIdx.x * kQueryRows;          // first row in those arrays
-    if (a.per > 0) {
+    if constexpr (std::is_same_v<Args, QueryPieces>) {
         const int rows = a.per * kQueryRows;
         spec = reinterpret_cast<float*>(a.slot[blockIdx.x / a.per]);
         spread = spec + (long long)rows * a.nout;
