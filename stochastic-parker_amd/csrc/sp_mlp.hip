@@ -496,6 +496,31 @@ __device__ __forceinline__ void ensemble_column(const EnsembleArgs& e, long long
     e.spec[o] = mean;
 }
 
+// Four columns of the members' outputs: their mean spectrum; dist grows by the
+// members' distances from it.
+template <int M>
+__device__ __forceinline__ float4 ensemble_columns(const float4 (&y)[M], int members, float floor, float inv,
+                                                   float& dist) {
+    float4 mv;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        float sv[M];
+        float mean = 0.0f;
+#pragma unroll
+        for (int i = 0; i < M; ++i)
+            if (i < members) {
+                sv[i] = fmaxf(pow10f((&y[i].x)[k]) - floor, 0.0f);
+                mean += sv[i];
+            }
+        mean *= inv;
+#pragma unroll
+        for (int i = 0; i < M; ++i)
+            if (i < members) dist += fabsf(sv[i] - mean);
+        (&mv.x)[k] = mean;
+    }
+    return mv;
+}
+
 __global__ void __launch_bounds__(256) ensemble_kernel(EnsembleArgs e, int rows) {
     const int l16 = threadIdx.x & 15;
     const long long r = (long long)blockIdx.x * 16 + (threadIdx.x >> 4);
@@ -509,24 +534,7 @@ __global__ void __launch_bounds__(256) ensemble_kernel(EnsembleArgs e, int rows)
 #pragma unroll
             for (int i = 0; i < 8; ++i)
                 if (i < e.members) yv[i] = *reinterpret_cast<const float4*>(e.y[i] + base + c);
-            float4 mv;
-            float* mp = &mv.x;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                float sv[8];
-                float mean = 0.0f;
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    if (i < e.members) {
-                        sv[i] = fmaxf(pow10f((&yv[i].x)[k]) - e.floor, 0.0f);
-                        mean += sv[i];
-                    }
-                mean *= inv;
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    if (i < e.members) dist += fabsf(sv[i] - mean);
-                mp[k] = mean;
-            }
+            const float4 mv = ensemble_columns<8>(yv, e.members, e.floor, inv, dist);
             *reinterpret_cast<float4*>(e.spec + base + c) = mv;
         } else {
             for (int k = c; k < min(c + 4, e.nout); ++k) ensemble_column(e, base + k, inv, dist);

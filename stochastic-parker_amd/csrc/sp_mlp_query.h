@@ -115,23 +115,7 @@ __global__ void __launch_bounds__(kQueryThreads) mlp_query_kernel(Args a) {
 #pragma unroll
             for (int i = 0; i < M; ++i)
                 if (i < a.members) yv[i] = *reinterpret_cast<const float4*>(&y[i][r * LY + c]);
-            float mv[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                float sv[M], mean = 0.0f;
-#pragma unroll
-                for (int i = 0; i < M; ++i)
-                    if (i < a.members) {
-                        sv[i] = fmaxf(pow10f((&yv[i].x)[k]) - a.floor, 0.0f);
-                        mean += sv[i];
-                    }
-                mean *= inv;
-#pragma unroll
-                for (int i = 0; i < M; ++i)
-                    if (i < a.members) dist += fabsf(sv[i] - mean);
-                mv[k] = mean;
-            }
-            *reinterpret_cast<float4*>(spec + (r0 + r) * a.nout + c) = float4{mv[0], mv[1], mv[2], mv[3]};
+            *reinterpret_cast<float4*>(spec + (r0 + r) * a.nout + c) = ensemble_columns<M>(yv, a.members, a.floor, inv, dist);
         }
 #pragma unroll
         for (int o = 8; o > 0; o >>= 1) dist += __shfl_xor(dist, o, 16);
