@@ -1218,8 +1218,15 @@ int ensemble(void* const* nets, int32_t members, const float* x, int64_t rows, d
         fused = fused && fused_ok(n) && same_shape(n, h);
     }
     const int nin = h->cfg.nin, nout = h->cfg.nout;
+    // the one-launch kernel's blocks write results while others read their rows,
+    // which therefore must not share device memory
+    auto meets = [&](const float* out, int64_t per) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(x), b = reinterpret_cast<uintptr_t>(out);
+        return a < b + 4 * (uintptr_t)(rows * per) && b < a + 4 * (uintptr_t)(rows * nin);
+    };
     const bool small = fused && rows > 0 && rows <= kQueryRowsMax && (dev || rows <= chunk) &&
-                       2 * h->cfg.nhidden * members <= sp::mlp::kQueryThreads;
+                       2 * h->cfg.nhidden * members <= sp::mlp::kQueryThreads &&
+                       !(dev && (meets(spec, nout) || meets(spread, 1)));
     if (!dev && !small && !h->ens_spec) {
         MLP_HIP(hipMalloc(&h->ens_spec, 4 * (size_t)h->bmax * nout));
         MLP_HIP(hipMalloc(&h->ens_spread, 4 * (size_t)h->bmax));
