@@ -91,8 +91,26 @@ __device__ __forceinline__ PhiloxPtl philox_ptl(uint32_t c0, uint32_t c1, uint32
                      (uint32_t)p0 ^ (k1 + kPhiloxW1)};
 }
 
+// The particle's two counter words alone, for kernels whose registers are better
+// spent than on two more.
+struct PhiloxTags {
+    uint32_t c0, c1;
+};
+
+__device__ __forceinline__ void philox_take(PhiloxPtl& q, uint32_t c0, uint32_t c1, uint32_t c3, uint32_t k0,
+                                            uint32_t k1) {
+    q = philox_ptl(c0, c1, c3, k0, k1);
+}
+__device__ __forceinline__ void philox_take(PhiloxTags& q, uint32_t c0, uint32_t c1, uint32_t, uint32_t, uint32_t) {
+    q = PhiloxTags{c0, c1};
+}
+
 // philox4x32_10(c0, c1, step, c3, k0, k1) of the particle's words
-__device__ __forceinline__ U4 philox_step(const PhiloxPtl& q, uint32_t step, uint32_t k0, uint32_t k1) {
+__device__ __forceinline__ U4 philox_step(const PhiloxTags& q, uint32_t step, uint32_t c3, uint32_t k0,
+                                          uint32_t k1) {
+    return philox4x32_10(q.c0, q.c1, step, c3, k0, k1);
+}
+__device__ __forceinline__ U4 philox_step(const PhiloxPtl& q, uint32_t step, uint32_t, uint32_t k0, uint32_t k1) {
     const uint64_t s1 = (uint64_t)kPhiloxM1 * step;
     const uint64_t s0 = (uint64_t)kPhiloxM0 * ((uint32_t)(s1 >> 32) ^ q.k0);
     return philox_rounds<2>((uint32_t)s1 ^ q.a, q.b, (uint32_t)(s0 >> 32) ^ q.c, (uint32_t)s0,

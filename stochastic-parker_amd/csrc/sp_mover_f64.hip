@@ -23,6 +23,8 @@ struct PolicyF64 {
         m.p0_2mpi = kv.p0_2mpi;
         m.perp_mag = kv.perp_mag; m.perp_mom = kv.perp_mom;
     }
+    template <int NDIM, bool TI, int FX>
+    using Rng = PhiloxPtl;
     template <int NDIM, bool TI, int FX, int PPL>
     using Cache = f64::CellCache<NDIM == 3 && !TI && (FX & FX_DPP) == 0>;
     template <int NDIM, bool TI, int FX, class GC>

@@ -71,13 +71,14 @@ __device__ __forceinline__ void pin_constants(MoverParams& m) {
 }
 
 // Per-slot state of the particle a lane is pushing.
+template <class Rng>
 struct Slot {
     long long idx;                // particle index (-1: none)
     State s;
     double w, dtarget, dt_old;
     double dl[4];                 // the last step's increments (for the undo)
     int cf, nsp, pending;
-    PhiloxPtl rng;
+    Rng rng;
     uint32_t rstep;
     unsigned ksteps;              // steps of this particle in this launch
     bool resumed;
@@ -155,7 +156,8 @@ mover_kernel(MoverParams m0) {
     bool exhausted = false;
     // start on this die's part of the range, then help the other parts
     int part = (int)(xcc_id() % (unsigned)kParts), parts_done = 0;
-    Slot sl[PPL];
+    using Rng = typename Pol::template Rng<NDIM, TINTERP, FX>;
+    Slot<Rng> sl[PPL];
     typename Pol::Var var[PPL];
     typename Pol::template Cache<NDIM, TINTERP, FX, PPL> gc;   // slot 0's last records
     gc.invalidate();
@@ -167,7 +169,7 @@ mover_kernel(MoverParams m0) {
         sl[k].dl[0] = sl[k].dl[1] = sl[k].dl[2] = sl[k].dl[3] = 0.0;
         sl[k].cf = sl[k].nsp = 0;
         sl[k].pending = PEND_NONE;
-        sl[k].rng = PhiloxPtl{0u, 0u, 0u, 0u};
+        sl[k].rng = Rng{};
         sl[k].rstep = 0u;
         sl[k].ksteps = 0u;
         sl[k].resumed = false;
@@ -182,7 +184,7 @@ mover_kernel(MoverParams m0) {
 #pragma unroll
         for (int k = 0; k < PPL; ++k) {
             if (kServe > 0 && !serve) break;
-            Slot& q = sl[k];
+            Slot<Rng>& q = sl[k];
             const bool need = q.idx < 0 && !exhausted;
             const unsigned long long need_mask = __builtin_amdgcn_ballot_w64(need);
             if (!need_mask) continue;
@@ -221,8 +223,8 @@ mover_kernel(MoverParams m0) {
                         v = v < 0 ? 0 : (v >= m0.nvar ? m0.nvar - 1 : v);
                         Pol::set_var(m, var[k], m0.var[v]);
                     }
-                    q.rng = philox_ptl((uint32_t)m.P.i(PI_TAGI)[j], (uint32_t)m.P.i(PI_TAGS)[j], m.stream,
-                                       m.key0, m.key1);
+                    philox_take(q.rng, (uint32_t)m.P.i(PI_TAGI)[j], (uint32_t)m.P.i(PI_TAGS)[j], m.stream,
+                                m.key0, m.key1);
                     q.rstep = prstep[j];
                     q.dl[0] = q.dl[1] = q.dl[2] = q.dl[3] = 0.0;
                     q.ksteps = 0;
@@ -250,7 +252,7 @@ mover_kernel(MoverParams m0) {
         bool do_push[PPL], fixed[PPL];
 #pragma unroll
         for (int k = 0; k < PPL; ++k) {
-            Slot& q = sl[k];
+            Slot<Rng>& q = sl[k];
             do_push[k] = false;
             fixed[k] = false;
             if (q.idx < 0) continue;
@@ -410,7 +412,7 @@ mover_kernel(MoverParams m0) {
 #pragma unroll
             for (int k = 0; k < PPL; ++k) {
                 if (!do_push[k]) continue;
-                Slot& q = sl[k];
+                Slot<Rng>& q = sl[k];
                 q.rstep += 1u;
                 int v = q.nsp + 1;  // mod(nsteps_pushed + 1, nsteps_interval)
                 if ((unsigned)v >= (unsigned)m.nsteps_interval) v %= m.nsteps_interval;

@@ -502,7 +502,7 @@ __device__ __forceinline__ void dpp_terms(const MoverParams& m, const KF& kf, fl
 // the step of several particles per lane is one straight-line block.
 // With FX_LEAN (no magnetic-field dependence of kappa, no 2D out-of-plane
 // drift) the terms those flags zero are left out of the arithmetic.
-template <int NDIM, int FX>
+template <int NDIM, int FX, bool FLOOR_BRANCH>
 __device__ __forceinline__ void kappa_push(const MoverParams& m, const KF& kf, State& s,
                                            const float* f, bool fixed_dt, const float r[4],
                                            double d[4]) {
@@ -707,11 +707,11 @@ __device__ __forceinline__ void kappa_push(const MoverParams& m, const KF& kf, S
     } else {
         s.p += dp;
     }
-    // momentum floor: back out the increment, land on 0.25 p0.  Rare: in 2D a
-    // wave without such a particle skips the two differences and the selects
-    // (the branch costs the 3D FP16 step 2 %: 27.9 -> 28.5 ms, 5e6 particles).
+    // momentum floor: back out the increment, land on 0.25 p0.  Rare: with
+    // FLOOR_BRANCH a wave without such a particle skips the two differences and
+    // the selects.
     const bool low = s.p < m.p_floor;
-    if (NDIM == 3 || __builtin_amdgcn_ballot_w64(low)) {
+    if (!FLOOR_BRANCH || __builtin_amdgcn_ballot_w64(low)) {
         const double pback = s.p - dp;
         dp = low ? m.p_floor - pback : dp;
         s.p = low ? m.p_floor : s.p;
@@ -723,9 +723,9 @@ __device__ __forceinline__ void kappa_push(const MoverParams& m, const KF& kf, S
 }
 
 // (2u - 1) sqrt(3) in FP32 from one Philox block: u = r / (2^32 - 1).
-__device__ __forceinline__ void step_rands(const MoverParams& m, const PhiloxPtl& rng, uint32_t step,
-                                           float r[4]) {
-    const U4 u = philox_step(rng, step, m.key0, m.key1);
+template <class Rng>
+__device__ __forceinline__ void step_rands(const MoverParams& m, const Rng& rng, uint32_t step, float r[4]) {
+    const U4 u = philox_step(rng, step, m.stream, m.key0, m.key1);
     const float sc = (float)(2.0 * 1.7320508075688772 / 4294967295.0);
     const float of = -1.7320508075688772f;
     r[0] = (float)u.a * sc + of;
@@ -734,7 +734,7 @@ __device__ __forceinline__ void step_rands(const MoverParams& m, const PhiloxPtl
     r[3] = (float)u.d * sc + of;
 }
 
-template <int NDIM, bool TINTERP, int FX, bool HALF, class GC>
+template <int NDIM, bool TINTERP, int FX, bool HALF, bool FLOOR_BRANCH, class GC>
 __device__ __forceinline__ void gather_kappa_push(const MoverParams& m, const KF& kf, State& s,
                                                   bool fixed_dt, const float r[4], double d[4],
                                                   GC& gc) {
@@ -747,7 +747,7 @@ __device__ __forceinline__ void gather_kappa_push(const MoverParams& m, const KF
     else if constexpr (NDIM == 2 && HALF) gather_pair2<TINTERP>(m, I, rt, f, gc);
     else if constexpr (NDIM == 2) gather_cell2<TINTERP>(m, I.rx, I.ry, I.ix, I.iy, rt, f, gc);
     else gather_node3<TINTERP, HALF>(m, I, rt, f, gc);
-    kappa_push<NDIM, FX>(m, kf, s, f, fixed_dt, r, d);
+    kappa_push<NDIM, FX, FLOOR_BRANCH>(m, kf, s, f, fixed_dt, r, d);
 }
 
 }  // namespace f32

@@ -558,7 +558,7 @@ __device__ __forceinline__ void push(const MoverParams& m, State& s, const doubl
 // of the four words (particle_module.f90:3548-3550, :3589).
 __device__ __forceinline__ void step_rands(const MoverParams& m, const PhiloxPtl& rng, uint32_t step,
                                            double r[4]) {
-    const U4 u = philox_step(rng, step, m.key0, m.key1);
+    const U4 u = philox_step(rng, step, m.stream, m.key0, m.key1);
     const double sqrt3 = sqrt(3.0);
     r[0] = (2.0 * u01(u.a) - 1.0) * sqrt3;
     r[1] = (2.0 * u01(u.b) - 1.0) * sqrt3;
