@@ -312,9 +312,17 @@ int mover_grid(Ctx* c, long long n, int bpc = 0, int ppl = 1) {
     // blocks per CU for the FP32 movers on the 2048^2 snapshot (two for
     // FP64), two for the FP16-record mover on the 512^3 snapshot (-38 %
     // kernel time against one); SP_MOVER_BLOCKS_PER_CU overrides.
-    const int per_cu_default =
+    int per_cu_default =
         c->cfg.ndim == 3 ? (prec == SP_PREC_F32H ? kMoverBlocksPerCU3DH : kMoverBlocksPerCU3D)
                          : (prec == SP_PREC_F64 ? kMoverBlocksPerCU2D64 : kMoverBlocksPerCU2D);
+    // With an acceleration region the 3D FP16 mover's second block pays once it is
+    // filled: up to then some SIMDs hold two chains of steps, the longest among
+    // them, and others one.  64^3, one block / two: 1e5 particles 17.9 / 22.2 ms
+    // (another configuration 22.6 / 24.2), 1.3e5 19.3 / 22.4, 2e5 23.2 / 23.1, 8e5 57.5 /
+    // 43.3.  Without the region it depends on the configuration (1e5: 16.7 / 20.5 and
+    // 25.5 / 22.4).
+    if (c->cfg.ndim == 3 && prec == SP_PREC_F32H && c->cfg.acc_region_flag && n <= 2ll * 256 * c->ncu)
+        per_cu_default = 1;
     int per_cu = std::min(std::max(1, occ), per_cu_default);
     if (c->tuned_bpc > 0) per_cu = std::min(std::max(1, occ), c->tuned_bpc);
     if (const char* e = std::getenv("SP_MOVER_BLOCKS_PER_CU")) {
