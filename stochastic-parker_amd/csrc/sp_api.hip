@@ -68,6 +68,8 @@ struct Ctx {
     int device = 0;
     int ncu = 0;
     hipStream_t st = nullptr;
+    // a mover call's begin, push, end and push's end; before the last two are
+    // recorded, and in other calls, marks that the host waits for
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     long long nnodes = 0;
     int recw = 0;
@@ -96,7 +98,6 @@ struct Ctx {
     long long mover_calls = 0;
     // autotuned launch settings (0 / -1: not tuned) and the tuner's state copy
     int tuned_bpc = 0, tuned_sort_steps = -1;
-    hipEvent_t slot_ev[2] = {};            // last kernels of the two groups of pieces
     void* pbuf_save = nullptr;
     // batched parameter variants
     sp::KappaVar* dvar = nullptr;
@@ -362,10 +363,10 @@ hipError_t pipe_pieces(Ctx* c, long long count, Submit submit, Drain drain) {
     for (long long g = 0; g <= groups && e == hipSuccess; ++g) {
         if (g < groups) {
             e = submit(g * G, pieces(g), pin.slots() + (g & 1) * G);
-            if (e == hipSuccess && g + 1 < groups) e = hipEventRecord(c->slot_ev[g & 1], c->st);
+            if (e == hipSuccess && g + 1 < groups) e = hipEventRecord(c->ev[2 + (g & 1)], c->st);
         }
         if (g > 0 && e == hipSuccess) {
-            e = g < groups ? hipEventSynchronize(c->slot_ev[(g - 1) & 1]) : hipStreamSynchronize(c->st);
+            e = g < groups ? hipEventSynchronize(c->ev[2 + ((g - 1) & 1)]) : hipStreamSynchronize(c->st);
             if (e == hipSuccess) drain((g - 1) * G, pieces(g - 1), pin.slots() + ((g - 1) & 1) * G);
         }
     }
@@ -604,8 +605,6 @@ void destroy(Ctx* c) {
     free_dev(c->pbuf_save);
     for (auto& e : c->ev)
         if (e) (void)hipEventDestroy(e);
-    for (auto& e : c->slot_ev)
-        if (e) (void)hipEventDestroy(e);
     if (c->st) (void)hipStreamDestroy(c->st);
     delete c;
 }
@@ -672,7 +671,6 @@ int sp_ctx_create(const sp_config* cfg, void** out_ctx) {
     c->ncu = prop.multiProcessorCount;
     SP_HIP_C(hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking));
     for (auto& e : c->ev) SP_HIP_C(hipEventCreate(&e));
-    for (auto& e : c->slot_ev) SP_HIP_C(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     SP_HIP_C(hipMalloc(&c->ctr, sizeof(sp::Counters)));
     SP_HIP_C(hipMemsetAsync(c->ctr, 0, sizeof(sp::Counters), c->st));
     for (int i = 0; i < 2; ++i) {
@@ -1039,7 +1037,7 @@ bool may_order(const Ctx* c, long long n, long long lanes, int ppl, unsigned bud
            ppl == 1 && budget == 0u && n > lanes && n >= sp::kOrderSample && (wait || n <= 16 * lanes);
 }
 
-// With counts, the sample of predicted step counts, and slot_ev[0] behind it;
+// With counts, the sample of predicted step counts, and ev[2] behind it;
 // else the digits of the work order.
 hipError_t launch_order(Ctx* c, const sp::MoverParams& m, uint32_t* digit, float* counts) {
     const int fx = step_features(c->cfg), nd = c->cfg.ndim;
@@ -1047,7 +1045,7 @@ hipError_t launch_order(Ctx* c, const sp::MoverParams& m, uint32_t* digit, float
     if (c->cfg.precision == SP_PREC_F32H) e = sp::launch_order_f32h(m, false, fx, nd, digit, counts, c->st);
     else if (c->cfg.precision == SP_PREC_F32) e = sp::launch_order_f32(m, false, fx, nd, digit, counts, c->st);
     else e = sp::launch_order_f64(m, false, fx, nd, digit, counts, c->st);
-    return e == hipSuccess && counts ? hipEventRecord(c->slot_ev[0], c->st) : e;
+    return e == hipSuccess && counts ? hipEventRecord(c->ev[2], c->st) : e;
 }
 
 // The push of one interval: launches of the persistent mover over the
@@ -1085,7 +1083,7 @@ int mover_run(Ctx* c, double t0, double dtf, int num_fine_steps, int nsteps_inte
         bool wait, ordered = may_order(c, nrun, lanes, ppl, m.step_budget, wait);
         if (ordered) {
             if (!sampled) SP_HIP(launch_order(c, m, nullptr, pr->counts));
-            SP_HIP(hipEventSynchronize(c->slot_ev[0]));
+            SP_HIP(hipEventSynchronize(c->ev[2]));
             ordered = order_pays(pr->counts, (double)lanes, (double)nrun, wait) && sort_buffers(c) == SP_OK;
         }
         sampled = false;
