@@ -18,7 +18,8 @@
 // 38 us per step, 21 + 14: a hidden layer takes the first kernel about 3700
 // cycles, the time of each CU's 128 KiB of weights from L2 (35 B per clock) and
 // of the BF16 activations' way to memory; the second reads 512 KiB of operands
-// per CU from L2 at 27 B per clock.  Neither dealing the layers to the dies, nor
+// per CU at 27 B per clock (43 % of its requests hit L2: blocks on all dies wrote
+// them).  Neither dealing the layers to the dies, nor
 // streaming stores, nor other places for the fragments changed the sum of both.
 #pragma once
 
